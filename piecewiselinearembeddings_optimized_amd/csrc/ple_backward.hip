@@ -1127,6 +1127,15 @@ constexpr int kMfmaMaxBins = 96;   // three tiles of 32 bins
 // table loads a thread has in flight in the set-up (c4, the whole kernel:
 // 4 / 8 -> 203-204 us, 16 -> 209-211, 32 -> 213-215)
 constexpr int kTabLoads = 8;
+// Gradients of at least this many bytes stream (non-temporal loads): read
+// with plain loads they pass through the 256 MB memory-side cache, which then
+// holds neither x nor the bin indices when the next forward wants them (c4:
+// the forward after this kernel 137 -> 103 us, this kernel 199 -> 207, the
+// step 329 -> 301; 16384 x 512, d = 32: 395 -> 349; 8192 x 1024, d = 8: 225
+// -> 215).  Smaller ones leave room there, and lines that two groups'
+// workgroups share are better kept (3001 x 201, d = 24, 29 MB: 76 -> 79 us
+// when streamed; 30001 x 101, d = 8, 48 MB: no difference).
+constexpr int64_t kMfmaStreamBytes = 64 << 20;
 constexpr int kMfmaFinLanes = 4;   // lanes of a (feature, column) in the kernel's dW / db step
 // the set-up reads a group's iw and edges one entry a thread, and clears the
 // stages 16 bytes at a time
@@ -1158,7 +1167,8 @@ static_assert(kStageBytes % 16 == 0, "stages cleared in 16-byte stores");
 // LDS in wave order, and they go, like the sorted path's, to dW / db (one
 // chunk) or to the chunk partials.  Rows of D = 8 NQ columns (NQ = 1..4), at
 // most 32 NBT bins; bin indices are uint8.
-template <int GD, int NBT, int NQ>
+// NT: the gradient streams past the caches (see kMfmaStreamBytes).
+template <int GD, int NBT, int NQ, bool NT>
 __global__ __launch_bounds__(kMfmaBlock, 1) void ple_bwd_mfma_kernel(BwdArgs a) {
     constexpr int D = 8 * NQ;
     constexpr int D2 = 2 * D;
@@ -1240,7 +1250,7 @@ __global__ __launch_bounds__(kMfmaBlock, 1) void ple_bwd_mfma_kernel(BwdArgs a) 
                       ns > 0 ? static_cast<uint32_t>(ns - 1) * rowFb + static_cast<uint32_t>(gspan) : 0u);
 #pragma unroll
         for (int r = 0; r < NP; ++r) {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, poff[r], 0, 0);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, poff[r], 0, NT ? kCpolNT : 0);
             gq[p][r] = make_uint2(v[0], v[1]);
         }
         const int xs = tid / FS, xf = tid - xs * FS;
@@ -2202,14 +2212,20 @@ void launch_bwd(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t s, cons
     hipExtLaunchKernelGGL(kernel, grid, block, static_cast<uint32_t>(lds), s, t_slot.start, t_slot.stop, 0u, a);
 }
 
+template <int GD, int NBT, bool NT>
+void launch_mfma_nq(int nq, dim3 grid, size_t lds, hipStream_t s, const BwdArgs &a) {
+    switch (nq) {
+        case 1: launch_bwd((ple_bwd_mfma_kernel<GD, NBT, 1, NT>), grid, dim3(kMfmaBlock), lds, s, a); break;
+        case 2: launch_bwd((ple_bwd_mfma_kernel<GD, NBT, 2, NT>), grid, dim3(kMfmaBlock), lds, s, a); break;
+        case 3: launch_bwd((ple_bwd_mfma_kernel<GD, NBT, 3, NT>), grid, dim3(kMfmaBlock), lds, s, a); break;
+        default: launch_bwd((ple_bwd_mfma_kernel<GD, NBT, 4, NT>), grid, dim3(kMfmaBlock), lds, s, a); break;
+    }
+}
+
 template <int GD, int NBT>
 void launch_mfma(int nq, dim3 grid, size_t lds, hipStream_t s, const BwdArgs &a) {
-    switch (nq) {
-        case 1: launch_bwd((ple_bwd_mfma_kernel<GD, NBT, 1>), grid, dim3(kMfmaBlock), lds, s, a); break;
-        case 2: launch_bwd((ple_bwd_mfma_kernel<GD, NBT, 2>), grid, dim3(kMfmaBlock), lds, s, a); break;
-        case 3: launch_bwd((ple_bwd_mfma_kernel<GD, NBT, 3>), grid, dim3(kMfmaBlock), lds, s, a); break;
-        default: launch_bwd((ple_bwd_mfma_kernel<GD, NBT, 4>), grid, dim3(kMfmaBlock), lds, s, a); break;
-    }
+    if (a.N * a.F * a.D * 2 >= kMfmaStreamBytes) launch_mfma_nq<GD, NBT, true>(nq, grid, lds, s, a);
+    else launch_mfma_nq<GD, NBT, false>(nq, grid, lds, s, a);
 }
 
 // Lane-group width as a template argument (DPP reductions) for the 4- and
