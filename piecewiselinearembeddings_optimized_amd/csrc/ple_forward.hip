@@ -76,23 +76,60 @@ constexpr int kStoreUnroll = 4;
 
 enum : int { kEpiNone = 0, kEpiBias = 1, kEpiBiasRelu = 2, kEpiLin = 3, kEpiLinRelu = 4 };
 
-// OR of v over the U consecutive lanes of a row (first lane: lane - u); every
-// lane of the row receives it.  Power-of-two rows are aligned to U lanes.
-__device__ __forceinline__ uint32_t row_or(uint32_t v, int U, int lane, int u) {
-    if ((U & (U - 1)) == 0) {
-        for (int off = 1; off < U; off <<= 1) v |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), off));
-        return v;
+// The ReLU mask word of a row whose first column is this lane's (meaningful
+// in the lanes that start a word: m_shift == 0): the VEC pass bits of up to
+// 32 / VEC consecutive lanes of the row, lane j's at bit VEC j.  mbits: this
+// lane's pass bits; o_u: its place among the row's U lanes.  No LDS round
+// trips: a chain of one shuffle per lane of the row used to set the time of
+// the ReLU forwards (10007 x 37, 100 bins, d = 15: 131 -> 38 us; 16384 x 64,
+// 128 bins, d = 64: 78 -> 61 us; 16384 x 100, 64 bins, d = 32 under bf16
+// autocast: 62 -> 55 us).  One or two columns a lane: ballots, shifted to the
+// lane and masked to its row (interleaved for two).  Four: an OR over the
+// row's lanes by DPP -- aligned groups of a power of two reduce by XOR
+// partners, other rows take their next lanes' words one shift at a time.
+// Every lane of the wave takes part.
+template <int VEC>
+__device__ __forceinline__ uint32_t mask_word(uint32_t mbits, int U, int lane, int o_u, int m_shift) {
+    constexpr int L = 32 / VEC;   // lanes of a word
+    if constexpr (VEC == 1 || VEC == 2) {
+        const int nl = min(L, U - o_u);
+        const uint32_t fm = nl >= 32 ? ~0u : (1u << nl) - 1u;
+        uint32_t w = static_cast<uint32_t>(__ballot(mbits & 1u) >> lane) & fm;
+        if constexpr (VEC == 2) {
+            const uint32_t odd = static_cast<uint32_t>(__ballot(mbits & 2u) >> lane) & fm;
+            auto spread = [](uint32_t v) __attribute__((always_inline)) {   // bit j of the low half to bit 2 j
+                v = (v | (v << 8)) & 0x00FF00FFu;
+                v = (v | (v << 4)) & 0x0F0F0F0Fu;
+                v = (v | (v << 2)) & 0x33333333u;
+                return (v | (v << 1)) & 0x55555555u;
+            };
+            w = spread(w) | (spread(odd) << 1);
+        }
+        return w;
+    } else {
+        static_assert(VEC == 4, "columns a lane");
+        int v = static_cast<int>(mbits << m_shift);
+        if ((U & (U - 1)) == 0) {
+            if (U >= 2) v |= __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);    // quad_perm: xor 1
+            if (U >= 4) v |= __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);    // quad_perm: xor 2
+            if (U >= 8) v |= __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true);   // row_half_mirror
+            return static_cast<uint32_t>(v);
+        }
+        int acc = v;
+        const int steps = min(L, U) - 1;
+        for (int j = 1; j <= steps; ++j) {
+            v = __builtin_amdgcn_update_dpp(0, v, 0x130, 0xF, 0xF, true);                // wave_shl: the next lane's
+            acc |= o_u + j < U ? v : 0;
+        }
+        return static_cast<uint32_t>(acc);
     }
-    uint32_t acc = 0;
-    for (int j = 0; j < U; ++j) acc |= static_cast<uint32_t>(__shfl(static_cast<int>(v), lane - u + j));
-    return acc;
 }
 
 // One lane's VEC results of an output row (fp32 fma of prefix and fraction
 // times weight) rounded through Q, the epilogue applied, stored as OUT at
 // element `oi` of the output.  With ReLU the pass bits of the row's U lanes
 // (this one is lane o_u of them) are gathered into the row's mask words at
-// `mi`.  bvec / lwv: the lane's bias or linear0 weight (linear0 bias in bvec);
+// `mi`, each stored by its first lane.  bvec / lwv: the lane's bias or linear0 weight (linear0 bias in bvec);
 // xs: the sample's x (linear0).
 template <int Q, int OUT, int EPI, int VEC, bool NT = true>
 __device__ __forceinline__ void emit_segment(const FwdArgs &a, float (&r)[VEC], const float (&bvec)[VEC],
@@ -120,13 +157,8 @@ __device__ __forceinline__ void emit_segment(const FwdArgs &a, float (&r)[VEC], 
     if (row_ok) store_out<OUT, VEC, NT>(a.out, oi, r);
     if constexpr (RELU) {
         if (a.mask) {
-            const uint32_t w0 = row_or(m_word == 0 ? mbits << m_shift : 0u, U, lane, o_u);
-            const uint32_t w1 = a.MW > 1 ? row_or(m_word == 1 ? mbits << m_shift : 0u, U, lane, o_u) : 0u;
-            if (row_ok && o_u == 0) {
-                uint32_t *mp = a.mask + mi;
-                mp[0] = w0;
-                if (a.MW > 1) mp[1] = w1;
-            }
+            const uint32_t w = mask_word<VEC>(mbits, U, lane, o_u, m_shift);
+            if (row_ok && m_shift == 0) a.mask[mi + m_word] = w;
         }
     }
 }
@@ -782,6 +814,12 @@ bool plan_forward(int64_t N, int64_t F, int64_t B, int64_t D, int out_bytes, boo
             // fp32, keep two rounds: one costs them 3 us)
             if (out_bytes == 2) c = slots / pl.G;
             if (c < 1) c = 1;
+        } else {
+            // Small batches: the table-bytes rule would leave CUs idle, and
+            // an idle CU saves nothing (10007 x 37, 100 bins, d = 15: 100
+            // workgroups 38 us, one per CU 28; 1024 x 50, 48 bins, d = 24: 75
+            // workgroups 14.5 us, one per CU 11.1, two 15.6).
+            c = std::max<int64_t>(c, device_cu_count() / pl.G);
         }
     }
     const int64_t sw = kWave / fs;
