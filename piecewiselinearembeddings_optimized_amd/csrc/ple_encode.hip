@@ -14,12 +14,24 @@
 // b > 0 and x == e_b (both neighbouring clamps pass at their bounds) -- the
 // same two-term rule as the embedding's dx.
 //
-// Forward kernel: one workgroup per block of kEncRows samples.  Phase 1
-// computes (b, frac) of every (sample, feature) pair of the block into LDS;
-// phase 2 walks the output row in 16-byte groups -- each thread finds the
-// features of its columns once (binary search over the LDS column offsets)
-// and then writes them for every sample of the block, so each store
-// instruction covers 1 KiB of one row.
+// Both kernels: one workgroup per (group of FG adjacent features, chunk of
+// samples).  It keeps the group's edges and inverse widths in LDS (searched
+// in global memory, a wave's 64 pairs touch up to 64 lines a step, which cost
+// more than the searches) and walks its samples in blocks of R rows; a thread
+// searches up to kEncPairs pairs of a block side by side, their x loaded a
+// block ahead.
+//
+// Forward: (b, frac) of the block's pairs go to LDS, then the threads walk
+// the group's columns of a row in 16-byte vectors -- each finds the features
+// of its columns once a block and writes them for every row -- so a store
+// instruction covers 1 KiB of one row, and the next block is searched while
+// the stores drain.  Bound by those stores, with the table set-up before them:
+// 16384 x 128, 48 bins (403 MB written) 109 -> 91 us, 700 x 900, 100 bins 366
+// -> 56.  Backward: one or two elements of g per pair, each in a line of its
+// own, kEncPairs lines in flight a thread and past the caches (each line is
+// read once): 74 -> 50 us and 38 -> 24 there.
+
+#include <algorithm>
 
 #include "ple_device.h"
 #include "ple_internal.h"
@@ -27,15 +39,20 @@
 namespace ple {
 namespace {
 
-constexpr int kEncRows = 8;   // samples per workgroup
+constexpr int kEncBlock = 2 * kBlock;
+constexpr int kEncPairs = 4;    // pairs of a block a thread searches, at most
+constexpr int kEncBlockPairs = kEncPairs * kEncBlock;
+constexpr size_t kEncLdsTarget = 72 * 1024;   // two workgroups per CU
 
 struct EncArgs {
     const float *x, *edges, *iw;
     const int32_t *nbins, *offsets;
     const float *g;      // backward: grad_output [N, T]
     float *out;          // forward: [N, T]; backward: grad_x [N, F]
-    int64_t N;
+    int64_t N, NC;       // samples; samples a chunk
     int F, B, T;
+    int FG, G, C, R;     // features a group, groups, chunks, rows a block
+    int ro_edge, ro_iw, ro_nb, ro_off;   // LDS offsets (bytes); the (b, frac) pairs are first
 };
 
 __device__ __forceinline__ float enc_value(int k, int b, float frac) {
@@ -44,118 +61,338 @@ __device__ __forceinline__ float enc_value(int k, int b, float frac) {
     return k < b ? 1.0f : (k == b ? frac : 0.0f);
 }
 
-template <bool V4>
-__global__ __launch_bounds__(kBlock) void ple_encode_kernel(EncArgs a) {
+// The group's tables and its samples' bins, shared by the two kernels.
+// TBL: edges and inverse widths in LDS (else read from global memory, see
+// plan_encode).
+template <bool TBL>
+struct EncGroup {
+    const EncArgs &a;
+    int f0, nf;                  // first feature, features (with the next group's first ones: see the forward)
+    int64_t n_begin, n_end;
+    float *s_edge, *s_iw;
+    int *s_nb, *s_off;
+    float xv[kEncPairs];         // x of this thread's pairs of the next block
+
+    __device__ __forceinline__ EncGroup(const EncArgs &args, unsigned char *lds) : a(args) {
+        s_edge = reinterpret_cast<float *>(lds + a.ro_edge);
+        s_iw = reinterpret_cast<float *>(lds + a.ro_iw);
+        s_nb = reinterpret_cast<int *>(lds + a.ro_nb);
+        s_off = reinterpret_cast<int *>(lds + a.ro_off);
+    }
+    __device__ __forceinline__ bool init(int halo) {
+        int g, c;
+        if (!decode_tile(blockIdx.x, a.G, a.C, g, c)) return false;
+        f0 = g * a.FG;
+        nf = min(a.F, f0 + a.FG + halo) - f0;
+        n_begin = static_cast<int64_t>(c) * a.NC;
+        n_end = min(a.N, n_begin + a.NC);
+        return n_begin < n_end;
+    }
+    // x of the pairs of the block at row n0: pair u of thread t is pair
+    // t + u kEncBlock of the block, sample-major (pairs past the block read x[0])
+    __device__ __forceinline__ void load_x(int64_t n0) {
+#pragma unroll
+        for (int u = 0; u < kEncPairs; ++u) {
+            const int i = threadIdx.x + u * kEncBlock;
+            const int s = i / nf;
+            const int64_t n = n0 + s;
+            xv[u] = a.x[s < a.R && n < n_end ? n * a.F + f0 + (i - s * nf) : 0];
+        }
+    }
+    __device__ __forceinline__ void stage() {
+        const int tid = threadIdx.x;
+        for (int i = tid; i < nf; i += kEncBlock) {
+            s_nb[i] = clamp_nbins(a.nbins[f0 + i], a.B);
+            s_off[i] = a.offsets[f0 + i];
+        }
+        if (tid == 0) s_off[nf] = f0 + nf < a.F ? a.offsets[f0 + nf] : a.T;
+        if constexpr (TBL) {
+            auto copy = [&](float *dst, const float *src, int count) __attribute__((always_inline)) {
+                for (int i0 = tid; i0 < count; i0 += 8 * kEncBlock) {
+                    float v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = src[min(i0 + u * kEncBlock, count - 1)];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (i0 + u * kEncBlock < count) dst[i0 + u * kEncBlock] = v[u];
+                }
+            };
+            copy(s_edge, a.edges + static_cast<int64_t>(f0) * (a.B + 1), nf * (a.B + 1));
+            copy(s_iw, a.iw + static_cast<int64_t>(f0) * a.B, nf * a.B);
+        }
+        __syncthreads();
+    }
+    __device__ __forceinline__ const float *edge_row(int fl) const {
+        if constexpr (TBL) return s_edge + fl * (a.B + 1);
+        else return a.edges + static_cast<int64_t>(f0 + fl) * (a.B + 1);
+    }
+    __device__ __forceinline__ const float *iw_row(int fl) const {
+        if constexpr (TBL) return s_iw + fl * a.B;
+        else return a.iw + static_cast<int64_t>(f0 + fl) * a.B;
+    }
+    // find_bin of the thread's pairs, a step of every search at a time
+    __device__ __forceinline__ void find(int (&fl)[kEncPairs], int (&b)[kEncPairs]) const {
+        int lo[kEncPairs], hi[kEncPairs], n[kEncPairs];
+        const float *e[kEncPairs];
+#pragma unroll
+        for (int u = 0; u < kEncPairs; ++u) {
+            fl[u] = static_cast<int>((threadIdx.x + u * kEncBlock) % static_cast<unsigned>(nf));
+            n[u] = s_nb[fl[u]];
+            e[u] = edge_row(fl[u]);
+            lo[u] = 0;
+            hi[u] = n[u] + 1;
+        }
+        const int steps = 32 - __clz(a.B + 1);
+        for (int t = 0; t < steps; ++t) {
+#pragma unroll
+            for (int u = 0; u < kEncPairs; ++u) {
+                const int mid = (lo[u] + hi[u]) >> 1;
+                const bool live = lo[u] < hi[u];
+                const bool below = xv[u] < e[u][min(mid, n[u])];
+                hi[u] = live && below ? mid : hi[u];
+                lo[u] = live && !below ? mid + 1 : lo[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kEncPairs; ++u) b[u] = clamp_bin(lo[u] - 1, n[u]);
+    }
+};
+
+// V4: 16-byte stores (T a multiple of 4).  A group owns the vectors whose
+// first column is one of its features'; such a vector may end in up to three
+// features of the next group, which this one searches too.
+template <bool V4, bool TBL>
+__global__ __launch_bounds__(kEncBlock) void ple_encode_kernel(EncArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
-    const int F = a.F, B = a.B, T = a.T;
-    int *s_off = reinterpret_cast<int *>(lds);                 // [F + 1] column offsets
-    int *s_bin = s_off + F + 1;                                // [kEncRows][F]
-    float *s_frac = reinterpret_cast<float *>(s_bin + kEncRows * F);
-    const int tid = threadIdx.x;
-    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kEncRows;
-    const int ns = static_cast<int>(min(static_cast<int64_t>(kEncRows), a.N - n0));
-
-    for (int i = tid; i < F; i += kBlock) s_off[i] = a.offsets[i];
-    if (tid == 0) s_off[F] = T;
-    for (int i = tid; i < ns * F; i += kBlock) {
-        const int s = i / F;
-        const int f = i - s * F;
-        const float v = a.x[(n0 + s) * F + f];
-        const int n = clamp_nbins(a.nbins[f], B);
-        const float *e = a.edges + static_cast<int64_t>(f) * (B + 1);
-        const int b = find_bin(v, e, n);
-        s_bin[i] = b;
-        s_frac[i] = (v - e[b]) * a.iw[static_cast<int64_t>(f) * B + b];
-    }
-    __syncthreads();
-
     constexpr int W = V4 ? 4 : 1;
-    for (int p0 = tid * W; p0 < T; p0 += kBlock * W) {
-        // feature of column p0: last f with off[f] <= p0
-        int lo = 0, hi = F;          // invariant: off[lo] <= p0 < off[hi]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (s_off[mid] <= p0) lo = mid;
-            else hi = mid;
-        }
-        int fq[W], kq[W];
-        int f = lo;
+    uint2 *s_pair = reinterpret_cast<uint2 *>(lds);   // [R][nf] {bin, frac bits}
+    EncGroup<TBL> gr(a, lds);
+    if (!gr.init(W - 1)) return;
+    const int tid = threadIdx.x;
+    const int nf = gr.nf, T = a.T;
+    gr.load_x(gr.n_begin);
+    gr.stage();
+    const int nown = min(a.F - gr.f0, a.FG);
+    const int c_begin = gr.f0 == 0 ? 0 : max(0, (gr.s_off[0] + W - 1) / W * W);
+    const int c_end = gr.f0 + nown == a.F ? T : min(T, gr.s_off[nown]);
+    // short rows: several rows side by side, sets of threads taking rows in turn
+    const int vecs = max(1, (c_end - c_begin + W - 1) / W);
+    const int sets = max(1, kEncBlock / vecs);
+    const int s0 = sets > 1 ? tid / vecs : 0;
+    const int v0 = sets > 1 ? (s0 < sets ? tid - s0 * vecs : vecs) : tid;   // (vecs: past the columns)
+
+    for (int64_t n0 = gr.n_begin; n0 < gr.n_end; n0 += a.R) {
+        const int ns = static_cast<int>(min(static_cast<int64_t>(a.R), gr.n_end - n0));
+        int fl[kEncPairs], b[kEncPairs];
+        gr.find(fl, b);
 #pragma unroll
-        for (int j = 0; j < W; ++j) {
-            const int p = min(p0 + j, T - 1);
-            while (f + 1 < F && p >= s_off[f + 1]) ++f;
-            fq[j] = f;
-            kq[j] = p - s_off[f];
+        for (int u = 0; u < kEncPairs; ++u) {
+            const int i = tid + u * kEncBlock;
+            const float frac = (gr.xv[u] - gr.edge_row(fl[u])[b[u]]) * gr.iw_row(fl[u])[b[u]];
+            if (i < ns * nf) s_pair[i] = make_uint2(static_cast<uint32_t>(b[u]), __float_as_uint(frac));
         }
-        for (int s = 0; s < ns; ++s) {
-            float v[W];
+        if (n0 + a.R < gr.n_end) gr.load_x(n0 + a.R);
+        __syncthreads();
+
+        for (int p0 = c_begin + v0 * W; p0 < c_end; p0 += kEncBlock * W) {
+            // feature of column p0: the last f with off[f] <= p0
+            int lo = 0, hi = nf;          // invariant: off[lo] <= p0 < off[hi]
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (gr.s_off[mid] <= p0) lo = mid;
+                else hi = mid;
+            }
+            int fq[W], kq[W];
+            int f = lo;
 #pragma unroll
-            for (int j = 0; j < W; ++j) v[j] = enc_value(kq[j], s_bin[s * F + fq[j]], s_frac[s * F + fq[j]]);
-            store_out<PLE_DTYPE_F32, W>(a.out, (n0 + s) * T + p0, v);
+            for (int j = 0; j < W; ++j) {
+                const int p = min(p0 + j, T - 1);
+                while (f + 1 < nf && p >= gr.s_off[f + 1]) ++f;
+                fq[j] = f;
+                kq[j] = p - gr.s_off[f];
+            }
+            // the first and last columns' features cover the vector unless a
+            // narrower feature lies between them
+            const bool two = !V4 || ((fq[W / 2] == fq[0] || fq[W / 2] == fq[W - 1]) &&
+                                     (fq[W > 1 ? 1 : 0] == fq[0] || fq[W > 1 ? 1 : 0] == fq[W - 1]));
+            const uint2 *first = s_pair + fq[0], *last = s_pair + fq[W - 1];
+            for (int s = s0; s < ns; s += sets) {
+                float v[W];
+                const uint2 pf = first[s * nf];
+                const uint2 pl = V4 ? last[s * nf] : pf;
+#pragma unroll
+                for (int j = 0; j < W; ++j) {
+                    const uint2 p = fq[j] == fq[0] ? pf : pl;
+                    v[j] = enc_value(kq[j], static_cast<int>(p.x), __uint_as_float(p.y));
+                }
+                if (!two) {
+#pragma unroll
+                    for (int j = 0; j < W; ++j) {
+                        const uint2 p = s_pair[s * nf + fq[j]];
+                        v[j] = enc_value(kq[j], static_cast<int>(p.x), __uint_as_float(p.y));
+                    }
+                }
+                store_out<PLE_DTYPE_F32, W>(a.out, (n0 + s) * T + p0, v);
+            }
         }
+        __syncthreads();
     }
 }
 
-// One thread per (sample, feature) pair.
-__global__ __launch_bounds__(kBlock) void ple_encode_backward_kernel(EncArgs a) {
+// One thread per (sample, feature) pair, everything from global memory: small
+// calls, whose time is the round trips of one pair (3000 x 5, 256 bins: 3.8
+// us against 8.6 with staged tables; 5759 x 84, 21 bins: 9.5 against 11.1;
+// 100000 x 6, 100 bins: 23.8 against 20.6, 700 x 900: 37.6 against 23.7).
+constexpr int64_t kEncSmallPairs = 1 << 19;
+__global__ __launch_bounds__(kBlock) void ple_encode_backward_small_kernel(EncArgs a) {
     const int F = a.F, B = a.B, T = a.T;
-    const int64_t pairs = a.N * F;
-    for (int64_t p = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; p < pairs;
-         p += static_cast<int64_t>(gridDim.x) * kBlock) {
-        const int64_t n = p / F;
-        const int f = static_cast<int>(p - n * F);
-        const float v = a.x[p];
-        const int nb = clamp_nbins(a.nbins[f], B);
-        const float *e = a.edges + static_cast<int64_t>(f) * (B + 1);
-        const float *iw = a.iw + static_cast<int64_t>(f) * B;
-        const int b = find_bin(v, e, nb);
-        // column of component b; columns outside [0, T) (offsets that do not
-        // match n_bins) read nothing
-        const int c = a.offsets[f] + b;
-        const float *grow = a.g + n * T;
-        float r = (c >= 0 && c < T) ? grow[c] * iw[b] : 0.0f;
-        if (b > 0 && v == e[b] && c - 1 >= 0 && c - 1 < T) r = fmaf(grow[c - 1], iw[b - 1], r);
-        a.out[p] = r;
+    const int64_t p = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (p >= a.N * F) return;
+    const int64_t n = p / F;
+    const int f = static_cast<int>(p - n * F);
+    const float v = a.x[p];
+    const int nb = clamp_nbins(a.nbins[f], B);
+    const float *e = a.edges + static_cast<int64_t>(f) * (B + 1);
+    const float *iw = a.iw + static_cast<int64_t>(f) * B;
+    const int b = find_bin(v, e, nb);
+    // column of component b; columns outside [0, T) (offsets that do not
+    // match n_bins) read nothing
+    const int c = a.offsets[f] + b;
+    const float *grow = a.g + n * T;
+    float r = (c >= 0 && c < T) ? grow[c] * iw[b] : 0.0f;
+    if (b > 0 && v == e[b] && c - 1 >= 0 && c - 1 < T) r = fmaf(grow[c - 1], iw[b - 1], r);
+    a.out[p] = r;
+}
+
+template <bool TBL>
+__global__ __launch_bounds__(kEncBlock) void ple_encode_backward_kernel(EncArgs a) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    EncGroup<TBL> gr(a, lds);
+    if (!gr.init(0)) return;
+    const int nf = gr.nf, T = a.T;
+    gr.load_x(gr.n_begin);
+    gr.stage();
+    for (int64_t n0 = gr.n_begin; n0 < gr.n_end; n0 += a.R) {
+        const int ns = static_cast<int>(min(static_cast<int64_t>(a.R), gr.n_end - n0));
+        int fl[kEncPairs], b[kEncPairs];
+        gr.find(fl, b);
+        float r[kEncPairs];
+        int64_t at[kEncPairs];
+        bool ok[kEncPairs], edge[kEncPairs];
+#pragma unroll
+        for (int u = 0; u < kEncPairs; ++u) {
+            const int i = threadIdx.x + u * kEncBlock;
+            ok[u] = i < ns * nf;
+            // column of component b; columns outside [0, T) (offsets that do
+            // not match n_bins) read nothing
+            const int c = gr.s_off[fl[u]] + b[u];
+            const int64_t n = n0 + i / nf;
+            at[u] = n * T + c;
+            edge[u] = ok[u] && b[u] > 0 && gr.xv[u] == gr.edge_row(fl[u])[b[u]] && c - 1 >= 0 && c - 1 < T;
+            const bool in = ok[u] && c >= 0 && c < T;
+            const float gv = __builtin_nontemporal_load(a.g + (in ? at[u] : 0));
+            r[u] = in ? gv * gr.iw_row(fl[u])[b[u]] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < kEncPairs; ++u)
+            if (edge[u]) r[u] = fmaf(a.g[at[u] - 1], gr.iw_row(fl[u])[b[u] - 1], r[u]);
+        if (n0 + a.R < gr.n_end) gr.load_x(n0 + a.R);
+#pragma unroll
+        for (int u = 0; u < kEncPairs; ++u) {
+            const int i = threadIdx.x + u * kEncBlock;
+            const int s = i / nf;
+            if (ok[u]) a.out[(n0 + s) * a.F + gr.f0 + (i - s * nf)] = r[u];
+        }
     }
 }
 
-size_t enc_lds_bytes(int F) {
-    return sizeof(int) * (F + 1) + (sizeof(int) + sizeof(float)) * static_cast<size_t>(kEncRows) * F;
+// Features a group: as many as two workgroups' LDS a CU hold (fewer where the
+// samples alone do not fill the CUs); chunks: one round of workgroups; rows a
+// block: kEncPairs pairs a thread.  halo: further features a group searches.
+// False: a single feature's tables do not fit LDS; then they stay in global
+// memory.
+bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
+    const int cus = device_cu_count();
+    const size_t pair_bytes = forward ? 8 * static_cast<size_t>(kEncBlockPairs) : 0;
+    const size_t per_f = 4 * (2 * static_cast<size_t>(a.B) + 3);   // edges, inverse widths, bin count, offset
+    const size_t room = kEncLdsTarget - pair_bytes - 64;
+    const bool tbl = per_f * (1 + halo) <= room;
+    int64_t fg = tbl ? static_cast<int64_t>(room / per_f) - halo : 512;
+    fg = std::min<int64_t>(fg, a.F);
+    const int64_t rows = (a.N + 15) / 16;
+    while (fg > 16 && (a.F + fg - 1) / fg * rows < cus) fg = (fg + 1) / 2;
+    a.FG = static_cast<int>(std::max<int64_t>(1, fg));
+    a.G = (a.F + a.FG - 1) / a.FG;
+    const int nfh = std::min(a.F, a.FG + halo);
+    a.R = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kEncBlockPairs / nfh, (a.N * a.G + cus - 1) / cus)));
+    int64_t c = (2 * static_cast<int64_t>(cus) + a.G - 1) / a.G;
+    c = std::max<int64_t>(1, std::min<int64_t>(c, (a.N + a.R - 1) / a.R));
+    a.NC = ((a.N + c - 1) / c + a.R - 1) / a.R * a.R;
+    a.C = static_cast<int>((a.N + a.NC - 1) / a.NC);
+    size_t off = forward ? 8 * static_cast<size_t>(a.R) * nfh : 0;
+    auto take = [&](int &field, size_t bytes) {
+        field = static_cast<int>(off);
+        off = align_up(off + bytes, 16);
+    };
+    take(a.ro_edge, tbl ? 4 * static_cast<size_t>(nfh) * (a.B + 1) : 0);
+    take(a.ro_iw, tbl ? 4 * static_cast<size_t>(nfh) * a.B : 0);
+    take(a.ro_nb, 4 * static_cast<size_t>(nfh));
+    take(a.ro_off, 4 * static_cast<size_t>(nfh + 1));
+    lds = off;
+    return tbl;
+}
+
+// The most features the encoding takes.
+constexpr int kEncMaxFeatures = 2409;
+
+EncArgs enc_args(const EncodeRequest &r) {
+    EncArgs a{};
+    a.x = r.x; a.edges = r.edges; a.iw = r.iw; a.nbins = r.nbins; a.offsets = r.offsets;
+    a.g = r.g; a.out = r.out;
+    a.N = r.N; a.F = static_cast<int>(r.F); a.B = static_cast<int>(r.B); a.T = static_cast<int>(r.T);
+    return a;
+}
+
+template <typename K>
+int enc_launch(K kernel, const EncArgs &a, size_t lds, hipStream_t s) {
+    const int64_t grid = kNumXcd * tiles_per_xcd(a.G, a.C);
+    if (grid > INT32_MAX) return PLE_E_TOO_LARGE;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kEncBlock), lds, s, a);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? PLE_OK : static_cast<int>(e);
 }
 
 }  // namespace
 
 int encode_run(const EncodeRequest &r) {
     if (r.T < 1 || r.T > INT32_MAX / 2) return PLE_E_TOO_LARGE;
-    const size_t lds = enc_lds_bytes(static_cast<int>(r.F));
-    if (lds > kLdsMax) return PLE_E_UNSUPPORTED;
-    EncArgs a{};
-    a.x = r.x; a.edges = r.edges; a.iw = r.iw; a.nbins = r.nbins; a.offsets = r.offsets;
-    a.out = r.out;
-    a.N = r.N; a.F = static_cast<int>(r.F); a.B = static_cast<int>(r.B); a.T = static_cast<int>(r.T);
-    const int64_t blocks = (r.N + kEncRows - 1) / kEncRows;
-    if (blocks > INT32_MAX) return PLE_E_TOO_LARGE;
+    if (r.F > kEncMaxFeatures) return PLE_E_UNSUPPORTED;
+    EncArgs a = enc_args(r);
     const bool v4 = r.T % 4 == 0 && reinterpret_cast<uintptr_t>(r.out) % 16 == 0;
-    if (v4) hipLaunchKernelGGL(ple_encode_kernel<true>, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), lds, r.stream, a);
-    else hipLaunchKernelGGL(ple_encode_kernel<false>, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), lds, r.stream, a);
-    const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? PLE_OK : static_cast<int>(e);
+    size_t lds;
+    const bool tbl = plan_encode(a, v4 ? 3 : 0, true, lds);
+    if (v4) {
+        return tbl ? enc_launch(ple_encode_kernel<true, true>, a, lds, r.stream)
+                   : enc_launch(ple_encode_kernel<true, false>, a, lds, r.stream);
+    }
+    return tbl ? enc_launch(ple_encode_kernel<false, true>, a, lds, r.stream)
+               : enc_launch(ple_encode_kernel<false, false>, a, lds, r.stream);
 }
 
 int encode_backward_run(const EncodeRequest &r) {
     if (r.T < 1 || r.T > INT32_MAX / 2) return PLE_E_TOO_LARGE;
-    EncArgs a{};
-    a.x = r.x; a.edges = r.edges; a.iw = r.iw; a.nbins = r.nbins; a.offsets = r.offsets;
-    a.g = r.g; a.out = r.out;
-    a.N = r.N; a.F = static_cast<int>(r.F); a.B = static_cast<int>(r.B); a.T = static_cast<int>(r.T);
-    const int64_t pairs = r.N * r.F;
-    int64_t blocks = (pairs + kBlock - 1) / kBlock;
-    const int64_t cap = static_cast<int64_t>(device_cu_count()) * 32;
-    if (blocks > cap) blocks = cap;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(ple_encode_backward_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, r.stream, a);
-    const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? PLE_OK : static_cast<int>(e);
+    EncArgs a = enc_args(r);
+    if (r.N * r.F < kEncSmallPairs) {
+        const int64_t blocks = (r.N * r.F + kBlock - 1) / kBlock;
+        hipLaunchKernelGGL(ple_encode_backward_small_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0,
+                           r.stream, a);
+        const hipError_t e = hipGetLastError();
+        return e == hipSuccess ? PLE_OK : static_cast<int>(e);
+    }
+    size_t lds;
+    const bool tbl = plan_encode(a, 0, false, lds);
+    return tbl ? enc_launch(ple_encode_backward_kernel<true>, a, lds, r.stream)
+               : enc_launch(ple_encode_backward_kernel<false>, a, lds, r.stream);
 }
 
 }  // namespace ple

@@ -1,0 +1,65 @@
+"""Dense encoding kernels at the edges of their plan.
+
+Feature groups (the tables of all features do not fit one workgroup), vectors
+that end in the next group's features (single-bin features at every place),
+row lengths that are not a multiple of four, rows shorter than a workgroup,
+blocks with a remainder, tables too large for LDS, and both sides of the pair
+count where the backward changes kernels.  Forward: bitwise against the closed
+form in fp32; backward: the fp32 bar around the float64 closed form.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ple_oracle as po
+from piecewiselinearembeddings_optimized_amd import workloads
+from tests.ple_cases import FP32_ATOL, FP32_RTOL, close_scaled
+
+pytestmark = pytest.mark.gpu
+
+# n, n_bins per feature
+CASES = {
+    "one_row": (1, [1, 2, 3, 4, 5]),
+    "short_rows": (5003, [3, 1]),
+    "singles": (77, [1] * 203),
+    "groups": (130, [1 + (7 * j) % 97 for j in range(400)]),
+    "groups_of_four": (97, [4 * (1 + j % 24) for j in range(400)]),
+    "singles_between_groups": (33, [96 if j % 5 else 1 for j in range(401)]),
+    "beyond_lds": (8200, [9001] + [1 + j % 3 for j in range(63)]),
+    "below_small_limit": (16383, [1 + j % 9 for j in range(32)]),
+    "at_small_limit": (16384, [1 + j % 9 for j in range(32)]),
+    "grouped_backward": (2700, [1 + (5 * j) % 60 for j in range(200)]),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_encode_groups(name):
+    assert torch.cuda.is_available(), "HIP device required"
+    import piecewiselinearembeddings_optimized_amd  # noqa: F401  (registers the ops)
+
+    ops = torch.ops.rtdl_num_embeddings_cuda
+    n, counts = CASES[name]
+    f = len(counts)
+    rng = np.random.default_rng(n)
+    bins = [np.unique(rng.uniform(-2, 2, c + 1).astype(np.float32)) for c in counts]
+    edges, inv_w, n_bins = workloads.pad_bins(bins)
+    x = rng.uniform(-2.5, 2.5, (n, f)).astype(np.float32)
+    rows = rng.integers(0, n, 200)
+    cols = rng.integers(0, f, 200)
+    x[rows, cols] = [bins[c][rng.integers(0, len(bins[c]))] for c in cols]     # on edges
+    offs = po.encoding_offsets(n_bins).astype(np.int32)
+    total = int(n_bins.sum())
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    tables = t(edges), t(inv_w), t(n_bins), t(offs)
+    g = rng.standard_normal((n, total)).astype(np.float32)
+    dx = ops.encode_backward(t(g), t(x), *tables)
+    ref, ref_abs = po.encoding_backward(g, x, edges, inv_w, n_bins)
+    ok, worst = close_scaled(dx.cpu().numpy(), ref, ref_abs, FP32_RTOL, FP32_ATOL)
+    assert ok, worst
+    x[rows[:20], cols[:20]] = np.nan
+    out = ops.encode(t(x), *tables, total).cpu().numpy()
+    exp = po.encoding_closed_form(x, edges, inv_w, n_bins, dtype=np.float32).astype(np.float32)
+    np.testing.assert_array_equal(out, exp)
