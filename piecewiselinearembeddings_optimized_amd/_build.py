@@ -95,13 +95,13 @@ def build_extension(verbose: bool = False) -> str:
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     incs = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], os.path.join(ROCM, "include"), INCLUDE]
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
-    src = os.path.join(CSRC, "ple_ops.cpp")
+    srcs = [os.path.join(CSRC, f) for f in ("ple_ops.cpp", "ple_autograd.cpp")]
     tmp = EXT_PATH + ".tmp"
     cmd = [
         os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
         "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
         *[f"-I{i}" for i in incs],
-        "-o", tmp, src,
+        "-o", tmp, *srcs,
         f"-L{PKG_DIR}", "-lple_hip",
         f"-L{torch_lib}", "-lc10", "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lamdhip64",
         "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}",
