@@ -9,7 +9,9 @@
 // `forward`: the same contract as the reference
 // (src/rtdl_num_embeddings_cuda/_autograd.py:9-96): the saved bin indices are
 // non-differentiable, grads are not materialised, and the backward operator
-// returns gradients for `x` and `weight` only.
+// returns gradients for `x` and `weight` only.  (Integer outputs, as the
+// indices and the ReLU pass bits are, are non-differentiable by their type;
+// compiled autograd refuses nodes that mark outputs so themselves.)
 //
 // `forward_with_bias`: additionally returns the bias gradient from the same
 // backward launch; `quant_dtype` is forwarded so the backward rounds the
@@ -111,7 +113,6 @@ struct Forward : torch::autograd::Function<Forward> {
         auto [out, idx] = op_forward().redispatch(below(ks), x, edges, iw, nbins, weight, output_dtype);
         ctx->save_for_backward({x, edges, iw, nbins, weight, idx});
         ctx->saved_data["need"] = need_bits(x, weight);
-        ctx->mark_non_differentiable({idx});
         ctx->set_materialize_grads(false);
         return {out, idx};
     }
@@ -147,7 +148,6 @@ struct ForwardWithBias : torch::autograd::Function<ForwardWithBias> {
         ctx->save_for_backward({x, edges, iw, nbins, weight, idx});
         ctx->saved_data["need"] = need_bits(x, weight, bias);
         ctx->saved_data["quant"] = static_cast<int64_t>(quant_dtype);
-        ctx->mark_non_differentiable({idx});
         ctx->set_materialize_grads(false);
         return {out, idx};
     }
@@ -190,7 +190,6 @@ struct ForwardEpilogue : torch::autograd::Function<ForwardEpilogue> {
         ctx->saved_data["relu"] = relu;
         // (the flag, not the mask's size: an empty batch saves an empty mask)
         ctx->saved_data["save_mask"] = save_mask;
-        ctx->mark_non_differentiable({idx, mask});
         ctx->set_materialize_grads(false);
         return {out, idx, mask};
     }
