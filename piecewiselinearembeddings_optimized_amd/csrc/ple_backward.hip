@@ -1966,8 +1966,11 @@ BwdPlan plan_backward(int64_t N, int64_t F, int64_t B, int64_t D, bool g_align16
     // matrix-core kernel, one workgroup per (group of FS features, chunk):
     // FS = 4 adjacent features where LDS holds their tables (2, 1 else),
     // chunks for a workgroup per CU (its eight waves fill the CU's two waves
-    // per SIMD) within the partials budget -- where that takes at most 8
-    // chunks: with more, shorter chunks' set-up, histogram merge and partials
+    // per SIMD; rounded down, as a few workgroups in a second round take as
+    // long as the first: operator alone, 8192 x 300, 64 bins, d = 24: 113 ->
+    // 79 us; 20000 x 170, d = 16: 147 -> 91; 5000 x 200, 90 bins, d = 16: 70
+    // -> 44) within the partials budget -- where that, rounded up, takes at
+    // most 8 chunks: with more, shorter chunks' set-up, histogram merge and partials
     // cost more than the sorted path (knob PLE_TUNE_BWD_MFMA: 1 never, 2
     // whenever the shape allows).
     const int mfma_knob = tuning(PLE_TUNE_BWD_MFMA);
@@ -1983,14 +1986,12 @@ BwdPlan plan_backward(int64_t N, int64_t F, int64_t B, int64_t D, bool g_align16
         geo.FS = fs;
         geo.G = static_cast<int>((F + fs - 1) / fs);
         const int64_t per_chunk = F * B * 2 * D * 4;
-        int64_t c = (static_cast<int64_t>(cus) + geo.G - 1) / geo.G;
         const int64_t budget_c = static_cast<int64_t>(kPartialBudget) / per_chunk;
-        if (c > budget_c) c = budget_c;
         // a few steps for every chunk
         const int64_t max_c = N / (static_cast<int64_t>(kMB) * 4 * (kMfmaWaves / fs));
-        if (c > max_c) c = max_c;
-        if (c < 1) c = 1;
-        if (c <= 8 || mfma_knob == 2) {
+        const int64_t c_up = std::min({(static_cast<int64_t>(cus) + geo.G - 1) / geo.G, budget_c, max_c});
+        if (c_up <= 8 || mfma_knob == 2) {
+            const int64_t c = std::max<int64_t>(std::min<int64_t>(cus / geo.G, c_up), 1);
             pl.mfma_nbt = static_cast<int>((B + 31) / 32);
             pl.mfma_nq = static_cast<int>(D / 8);
             pl.rb = kMfmaBlock;
@@ -2117,26 +2118,49 @@ BwdPlan plan_backward(int64_t N, int64_t F, int64_t B, int64_t D, bool g_align16
                     geo.BW = nw > 1 ? bw : static_cast<int>(B);
                     geo.NW = nw;
                     geo.G = static_cast<int>((F + best_fs - 1) / best_fs) * nw;
-                    geo.NT = kP / best_fs;
-                    geo.T = static_cast<int>((N + geo.NT - 1) / geo.NT);
                     geo.PM = PM;
                     geo.LGW = lgw;
                     // chunks of sub-tiles: as many workgroups as the CUs
                     // hold at once (registers allow two 256-thread or one
-                    // 512-thread workgroup per CU; LDS may allow fewer), so
-                    // that every workgroup starts in the first round, within
-                    // the partials budget.  More rounds (the
-                    // PLE_TUNE_BWD_WG_PER_CU knob) measured slower: each
-                    // workgroup stages its tables and writes its partials.
+                    // 512-thread workgroup per CU; LDS may allow fewer),
+                    // rounded down, so that every workgroup starts in the
+                    // first round, within the partials budget.  More rounds
+                    // (the PLE_TUNE_BWD_WG_PER_CU knob) measured slower: each
+                    // workgroup stages its tables and writes its partials,
+                    // and a count rounded up leaves a second round for a few
+                    // workgroups, which then takes as long as the first:
+                    // operator alone, 100 groups of 16384 x 100, 64 bins,
+                    // d = 32 (linear0 + ReLU, bf16 quantisation) 6 chunks
+                    // 159 us, 5 chunks 117; 40000 x 33, 128 bins, d = 48: 154
+                    // -> 95; 16384 x 300, 48 bins, d = 16: 212 -> 144; 1024 x
+                    // 600, 40 bins, d = 16: 54 -> 43.  The chunks' sub-tiles
+                    // are all of one size (whole 64-pair blocks), so that no
+                    // workgroup has one more than the others: 30000 x 70, 32
+                    // bins, d = 32: 102 -> 98 with both.  More chunks of less
+                    // than a full sub-tile gain nothing (10007 x 37, 100
+                    // bins, d = 15: 42.9 / 42.2 / 42.2 us at 1024 / 512 / 256
+                    // pairs) and cost up to a quarter (8192 x 24, 20 bins,
+                    // d = 12: 22 -> 27).
                     const int64_t per_chunk = F * B * 2 * D * 4;
                     const int resident = rb == kWideBlock ? 1 : static_cast<int>(std::min<size_t>(2, kLdsMax / best_lds));
                     const int wg_k = tuning(PLE_TUNE_BWD_WG_PER_CU);
-                    int64_t c = (static_cast<int64_t>(wg_k > 0 ? wg_k : resident) * cus + geo.G - 1) / geo.G;
+                    const int64_t slots = static_cast<int64_t>(wg_k > 0 ? wg_k : resident) * cus;
                     const int64_t budget_c = static_cast<int64_t>(kPartialBudget) / per_chunk;
-                    if (c > budget_c) c = budget_c;
-                    if (c > geo.T) c = geo.T;
-                    if (c < 1) c = 1;
-                    geo.SPC = static_cast<int>((geo.T + c - 1) / c);
+                    const int64_t nt_max = kP / best_fs;
+                    const int64_t t_full = std::max<int64_t>((N + nt_max - 1) / nt_max, 1);   // full sub-tiles
+                    // chunks of whole sub-tiles in a count rounded up: no
+                    // more than these, so that the partials of a shape (and
+                    // the shapes that a fixed workspace holds) never exceed
+                    // what that count needs
+                    int64_t c_cap = std::max<int64_t>(std::min({(slots + geo.G - 1) / geo.G, budget_c, t_full}), 1);
+                    const int64_t spc_cap = (t_full + c_cap - 1) / c_cap;
+                    c_cap = (t_full + spc_cap - 1) / spc_cap;
+                    const int64_t c = std::max<int64_t>(std::min(slots / geo.G, c_cap), 1);
+                    const int64_t per = std::max<int64_t>((N + c - 1) / c, 1);   // samples a chunk
+                    geo.SPC = static_cast<int>((per + nt_max - 1) / nt_max);
+                    const int64_t step = std::max(1, kWave / best_fs);
+                    geo.NT = static_cast<int>((per + geo.SPC * step - 1) / (geo.SPC * step) * step);
+                    geo.T = static_cast<int>((N + geo.NT - 1) / geo.NT);
                     pl.C = pl.Cd = (geo.T + geo.SPC - 1) / geo.SPC;
                     pl.NC = static_cast<int64_t>(geo.SPC) * geo.NT;
                     pl.geo = geo;
