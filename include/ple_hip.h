@@ -254,7 +254,8 @@ int ple_backward_epilogue_launch(const float *grad_output, const float *x, const
  *   1 (k < b), frac (k == b), 0 (k > b);   NaN x: all NaN.
  *   offsets         int32 [F], offsets[f] = sum_{j<f} n_bins[j]
  *   output          float32 [N, total_bins], total_bins = sum_f n_bins[f]
- * F * 8 * 8 + 4 bytes of per-feature tables must fit LDS (F <= 2500).
+ * At most 2409 features (PLE_E_UNSUPPORTED beyond; the backward has no such
+ * limit).
  */
 int ple_encode_launch(const float *x, const float *bin_edges, const float *inv_bin_widths,
                       const int32_t *n_bins, const int32_t *offsets, float *output, int64_t N,
@@ -266,6 +267,35 @@ int ple_encode_backward_launch(const float *grad_output, const float *x, const f
                                const float *inv_bin_widths, const int32_t *n_bins,
                                const int32_t *offsets, float *grad_x, int64_t N, int64_t F,
                                int64_t B, int64_t total_bins, void *stream);
+
+/*
+ * The launch plan of ple_encode_launch (backward 0) or
+ * ple_encode_backward_launch (backward 1) for a shape, without launching.
+ * `output` may be NULL (then taken as 16-byte aligned).  Returns the error the
+ * launch would return for the sizes, else fills `info`; all zeros: the
+ * backward of a small call, one thread per (sample, feature) pair.
+ *   features_per_group  adjacent features whose columns a workgroup writes
+ *   features_searched   features whose bins it searches: with 16-byte stores up
+ *                       to three more, whose columns share its last vector
+ *   groups, chunks      feature groups, sample chunks
+ *   rows_per_block      samples searched together
+ *   pairs_per_block     (sample, feature) pairs that the threads of a workgroup
+ *                       search together, at most: rows_per_block *
+ *                       features_searched never exceeds it
+ *   lds_tables          1: the group's edges and inverse widths are kept in LDS
+ */
+typedef struct ple_encode_plan_info {
+    int features_per_group;
+    int features_searched;
+    int groups;
+    int chunks;
+    int rows_per_block;
+    int pairs_per_block;
+    int lds_tables;
+    size_t lds_bytes;
+} ple_encode_plan_info_t;
+int ple_encode_plan_query(const void *output, int64_t N, int64_t F, int64_t B, int64_t total_bins,
+                          int backward, ple_encode_plan_info_t *info);
 
 /*
  * Planner overrides, for tuning sweeps and for tests that run every kernel

@@ -61,6 +61,21 @@ class BackwardPlanInfo(ctypes.Structure):
     ]
 
 
+class EncodePlanInfo(ctypes.Structure):
+    """``ple_encode_plan_info_t``: the dense encoding's launch plan for a shape."""
+
+    _fields_ = [
+        ("features_per_group", ctypes.c_int),
+        ("features_searched", ctypes.c_int),
+        ("groups", ctypes.c_int),
+        ("chunks", ctypes.c_int),
+        ("rows_per_block", ctypes.c_int),
+        ("pairs_per_block", ctypes.c_int),
+        ("lds_tables", ctypes.c_int),
+        ("lds_bytes", ctypes.c_size_t),
+    ]
+
+
 class PleError(RuntimeError):
     def __init__(self, code: int, message: str):
         super().__init__(f"{message} (code {code})")
@@ -100,6 +115,8 @@ def lib() -> ctypes.CDLL:
         L.ple_encode_launch.restype = i32
         L.ple_encode_backward_launch.argtypes = [p, p, p, p, p, p, p, i64, i64, i64, i64, p]
         L.ple_encode_backward_launch.restype = i32
+        L.ple_encode_plan_query.argtypes = [p, i64, i64, i64, i64, i32, ctypes.POINTER(EncodePlanInfo)]
+        L.ple_encode_plan_query.restype = i32
         L.ple_timing_start.argtypes, L.ple_timing_start.restype = [i32], i32
         L.ple_timing_stop.argtypes, L.ple_timing_stop.restype = [], i32
         L.ple_timing_read.argtypes = [i32, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int)]
@@ -178,6 +195,14 @@ def backward_plan(n: int, f: int, bmax: int, d: int, grad_dtype=torch.float32, q
     check(lib().ple_backward_plan_query(_ptr(grad_output), n, f, bmax, d, dtype_code(grad_dtype), dtype_code(q),
                                         1 if relu else 0, 1 if linear0 else 0, ctypes.byref(info)))
     return {name: getattr(info, name) for name, _ in BackwardPlanInfo._fields_}
+
+
+def encode_plan(n: int, f: int, bmax: int, total_bins: int, backward: bool = False, output=None) -> dict:
+    """``ple_encode_plan_query``: the plan an encoding (or its backward) of
+    this shape takes, as a dict of :class:`EncodePlanInfo`'s fields."""
+    info = EncodePlanInfo()
+    check(lib().ple_encode_plan_query(_ptr(output), n, f, bmax, total_bins, 1 if backward else 0, ctypes.byref(info)))
+    return {name: getattr(info, name) for name, _ in EncodePlanInfo._fields_}
 
 
 def backward(grad_output, x, bin_edges, inv_bin_widths, n_bins, weight, bin_indices, grad_x, grad_weight,

@@ -114,7 +114,7 @@ int check_common(int64_t N, int64_t F, int64_t B, int64_t D) {
 
 extern "C" {
 
-int ple_abi_version(void) { return (1 << 16) | 4; }
+int ple_abi_version(void) { return (1 << 16) | 5; }
 
 int ple_bin_index_bytes(int64_t max_n_bins) { return ple::idx_bytes_for(max_n_bins); }
 
@@ -366,6 +366,19 @@ int ple_encode_backward_launch(const float *grad_output, const float *x, const f
     r.N = N; r.F = F; r.B = B; r.T = total_bins;
     r.stream = static_cast<hipStream_t>(stream);
     return ple::encode_backward_run(r);
+}
+
+int ple_encode_plan_query(const void *output, int64_t N, int64_t F, int64_t B, int64_t total_bins,
+                          int backward, ple_encode_plan_info_t *info) {
+    const int rc = ple::check_common(N, F, B, 1);
+    if (rc != PLE_OK) return rc;
+    if (total_bins < 1 || N < 1) return PLE_E_BAD_SHAPE;
+    if (N > INT64_MAX / total_bins) return PLE_E_TOO_LARGE;
+    if (!info) return PLE_E_NULL_POINTER;
+    ple::EncodeRequest r{};
+    r.out = static_cast<float *>(const_cast<void *>(output));
+    r.N = N; r.F = F; r.B = B; r.T = total_bins;
+    return ple::encode_plan_info(r, backward != 0, info);
 }
 
 }  // extern "C"

@@ -308,9 +308,10 @@ __global__ __launch_bounds__(kEncBlock) void ple_encode_backward_kernel(EncArgs 
 
 // Features a group: as many as two workgroups' LDS a CU hold (fewer where the
 // samples alone do not fill the CUs); chunks: one round of workgroups; rows a
-// block: kEncPairs pairs a thread.  halo: further features a group searches.
-// False: a single feature's tables do not fit LDS; then they stay in global
-// memory.
+// block: kEncPairs pairs a thread; with the features that a row of a block has
+// never more than kEncBlockPairs, the pairs that the threads search.  halo:
+// further features a group searches.  False: a single feature's tables do not
+// fit LDS; then they stay in global memory.
 bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
     const int cus = device_cu_count();
     const size_t pair_bytes = forward ? 8 * static_cast<size_t>(kEncBlockPairs) : 0;
@@ -318,7 +319,7 @@ bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
     const size_t room = kEncLdsTarget - pair_bytes - 64;
     const bool tbl = per_f * (1 + halo) <= room;
     int64_t fg = tbl ? static_cast<int64_t>(room / per_f) - halo : 512;
-    fg = std::min<int64_t>(fg, a.F);
+    fg = std::min<int64_t>({fg, a.F, kEncBlockPairs - halo});
     const int64_t rows = (a.N + 15) / 16;
     while (fg > 16 && (a.F + fg - 1) / fg * rows < cus) fg = (fg + 1) / 2;
     a.FG = static_cast<int>(std::max<int64_t>(1, fg));
@@ -342,7 +343,7 @@ bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
     return tbl;
 }
 
-// The most features the encoding takes.
+// The most features the forward takes, part of its interface (ple_hip.h).
 constexpr int kEncMaxFeatures = 2409;
 
 EncArgs enc_args(const EncodeRequest &r) {
@@ -353,8 +354,13 @@ EncArgs enc_args(const EncodeRequest &r) {
     return a;
 }
 
+// Rows of whole 16-byte vectors.
+bool enc_vectors(const EncodeRequest &r) { return r.T % 4 == 0 && reinterpret_cast<uintptr_t>(r.out) % 16 == 0; }
+
 template <typename K>
-int enc_launch(K kernel, const EncArgs &a, size_t lds, hipStream_t s) {
+int enc_launch(K kernel, const EncArgs &a, int halo, size_t lds, hipStream_t s) {
+    // (plan_encode's bound: pairs past it would not be searched)
+    if (static_cast<int64_t>(a.R) * std::min(a.F, a.FG + halo) > kEncBlockPairs) return PLE_E_UNSUPPORTED;
     const int64_t grid = kNumXcd * tiles_per_xcd(a.G, a.C);
     if (grid > INT32_MAX) return PLE_E_TOO_LARGE;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kEncBlock), lds, s, a);
@@ -368,15 +374,16 @@ int encode_run(const EncodeRequest &r) {
     if (r.T < 1 || r.T > INT32_MAX / 2) return PLE_E_TOO_LARGE;
     if (r.F > kEncMaxFeatures) return PLE_E_UNSUPPORTED;
     EncArgs a = enc_args(r);
-    const bool v4 = r.T % 4 == 0 && reinterpret_cast<uintptr_t>(r.out) % 16 == 0;
+    const bool v4 = enc_vectors(r);
+    const int halo = v4 ? 3 : 0;
     size_t lds;
-    const bool tbl = plan_encode(a, v4 ? 3 : 0, true, lds);
+    const bool tbl = plan_encode(a, halo, true, lds);
     if (v4) {
-        return tbl ? enc_launch(ple_encode_kernel<true, true>, a, lds, r.stream)
-                   : enc_launch(ple_encode_kernel<true, false>, a, lds, r.stream);
+        return tbl ? enc_launch(ple_encode_kernel<true, true>, a, halo, lds, r.stream)
+                   : enc_launch(ple_encode_kernel<true, false>, a, halo, lds, r.stream);
     }
-    return tbl ? enc_launch(ple_encode_kernel<false, true>, a, lds, r.stream)
-               : enc_launch(ple_encode_kernel<false, false>, a, lds, r.stream);
+    return tbl ? enc_launch(ple_encode_kernel<false, true>, a, halo, lds, r.stream)
+               : enc_launch(ple_encode_kernel<false, false>, a, halo, lds, r.stream);
 }
 
 int encode_backward_run(const EncodeRequest &r) {
@@ -391,8 +398,27 @@ int encode_backward_run(const EncodeRequest &r) {
     }
     size_t lds;
     const bool tbl = plan_encode(a, 0, false, lds);
-    return tbl ? enc_launch(ple_encode_backward_kernel<true>, a, lds, r.stream)
-               : enc_launch(ple_encode_backward_kernel<false>, a, lds, r.stream);
+    return tbl ? enc_launch(ple_encode_backward_kernel<true>, a, 0, lds, r.stream)
+               : enc_launch(ple_encode_backward_kernel<false>, a, 0, lds, r.stream);
+}
+
+int encode_plan_info(const EncodeRequest &r, bool backward, ple_encode_plan_info_t *info) {
+    if (r.T < 1 || r.T > INT32_MAX / 2) return PLE_E_TOO_LARGE;
+    if (!backward && r.F > kEncMaxFeatures) return PLE_E_UNSUPPORTED;
+    *info = ple_encode_plan_info_t{};
+    if (backward && r.N * r.F < kEncSmallPairs) return PLE_OK;
+    EncArgs a = enc_args(r);
+    const int halo = !backward && enc_vectors(r) ? 3 : 0;
+    size_t lds;
+    info->lds_tables = plan_encode(a, halo, !backward, lds) ? 1 : 0;
+    info->features_per_group = a.FG;
+    info->features_searched = std::min(a.F, a.FG + halo);
+    info->groups = a.G;
+    info->chunks = a.C;
+    info->rows_per_block = a.R;
+    info->pairs_per_block = kEncBlockPairs;
+    info->lds_bytes = lds;
+    return PLE_OK;
 }
 
 }  // namespace ple

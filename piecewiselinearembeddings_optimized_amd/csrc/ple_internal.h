@@ -96,5 +96,8 @@ struct EncodeRequest {
 
 int encode_run(const EncodeRequest &r);
 int encode_backward_run(const EncodeRequest &r);
+// The plan encode_run / encode_backward_run would take (of the pointers only
+// the address of `out` counts).
+int encode_plan_info(const EncodeRequest &r, bool backward, ple_encode_plan_info_t *info);
 
 }  // namespace ple
