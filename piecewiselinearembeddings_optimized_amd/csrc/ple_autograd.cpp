@@ -24,7 +24,9 @@
 // `encode`: the gradient of `x` from `encode_backward`.
 //
 // The operators are called through the dispatcher on both ways, so fake
-// tensors, tracing and batched gradients see them.  Double backward and
+// tensors, tracing and batched gradients see them, and the backwards have no
+// state or side effects, so compiled autograd traces them into its graph
+// (is_traceable) instead of breaking it for a call in eager mode.  Double backward and
 // forward-mode derivatives are not implemented (as in the reference).
 
 #include <ATen/ATen.h>
@@ -106,6 +108,7 @@ int64_t need_bits(const T &...t) {
 Tensor if_bit(int64_t bits, int i, Tensor t) { return (bits >> i) & 1 ? std::move(t) : Tensor(); }
 
 struct Forward : torch::autograd::Function<Forward> {
+    static constexpr bool is_traceable = true;
     static variable_list forward(AutogradContext *ctx, DispatchKeySet ks, const Tensor &x, const Tensor &edges,
                                  const Tensor &iw, const Tensor &nbins, const Tensor &weight,
                                  at::ScalarType output_dtype) {
@@ -140,6 +143,7 @@ Tensors2 forward(DispatchKeySet ks, const Tensor &x, const Tensor &edges, const 
 }
 
 struct ForwardWithBias : torch::autograd::Function<ForwardWithBias> {
+    static constexpr bool is_traceable = true;
     static variable_list forward(AutogradContext *ctx, DispatchKeySet ks, const Tensor &x, const Tensor &edges,
                                  const Tensor &iw, const Tensor &nbins, const Tensor &weight, const Tensor &bias,
                                  at::ScalarType quant_dtype) {
@@ -177,6 +181,7 @@ Tensors2 forward_with_bias(DispatchKeySet ks, const Tensor &x, const Tensor &edg
 }
 
 struct ForwardEpilogue : torch::autograd::Function<ForwardEpilogue> {
+    static constexpr bool is_traceable = true;
     static variable_list forward(AutogradContext *ctx, DispatchKeySet ks, const Tensor &x, const Tensor &edges,
                                  const Tensor &iw, const Tensor &nbins, const Tensor &weight, const OptTensor &bias,
                                  const OptTensor &lin_weight, const OptTensor &lin_bias, bool relu, bool save_mask,
@@ -230,6 +235,7 @@ Tensors3 forward_epilogue(DispatchKeySet ks, const Tensor &x, const Tensor &edge
 }
 
 struct Encode : torch::autograd::Function<Encode> {
+    static constexpr bool is_traceable = true;
     static Tensor forward(AutogradContext *ctx, DispatchKeySet ks, const Tensor &x, const Tensor &edges,
                           const Tensor &iw, const Tensor &nbins, const Tensor &offsets, int64_t total_bins) {
         at::AutoDispatchBelowAutograd guard;

@@ -50,6 +50,55 @@ def test_compiled_autograd(op):
     assert [t.grad.shape for t in wrt] == [t.shape for t in wrt]
 
 
+def _one_graph_compiler(graphs):
+    """A compiler that takes whole graphs only, and notes the operator calls of each."""
+    from torch._dynamo.backends.common import aot_autograd
+
+    def compile_graph(gm, _example_inputs):
+        graphs.append([(str(n.target), [a for a in n.args if not isinstance(a, torch.fx.Node)])
+                       for n in gm.graph.nodes if "rtdl_num_embeddings_cuda" in str(n.target)])
+        return gm.forward
+
+    torch._dynamo.reset()
+    return torch.compile(backend=aot_autograd(fw_compiler=compile_graph), fullgraph=True)
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_compiled_autograd_is_one_graph(op):
+    from torch._dynamo import compiled_autograd
+
+    graphs = []
+    compiler = _one_graph_compiler(graphs)
+    out, wrt = _call(op)
+    with compiled_autograd._enable(compiler):
+        out.sum().backward()
+    backward = "encode_backward" if op == "encode" else op.replace("forward", "backward")
+    assert [[name for name, _ in g] for g in graphs] == [[f"rtdl_num_embeddings_cuda.{backward}.default"]]
+    assert [t.grad.shape for t in wrt] == [t.shape for t in wrt]
+
+
+def test_compiled_autograd_keeps_a_graph_per_option():
+    """The flags and the dtype a node saved are constants of its graph."""
+    from torch._dynamo import compiled_autograd
+
+    graphs = []
+    compiler = _one_graph_compiler(graphs)
+
+    def step(quant, relu, grad_bias):
+        x, edges, iw, nb = _meta(N, F), _meta(F, B + 1), _meta(F, B), _meta(F, dtype=torch.int32)
+        weight, bias = _meta(F, B, D, requires_grad=True), _meta(F, D, requires_grad=grad_bias)
+        out = _ops.forward_epilogue(x, edges, iw, nb, weight, bias, None, None, relu, True, quant)[0]
+        known = len(graphs)
+        with compiled_autograd._enable(compiler):
+            out.sum().backward()
+        return [args for g in graphs[known:] for _, args in g]
+
+    for quant, relu, grad_bias in [(torch.float32, True, True), (torch.bfloat16, True, True),
+                                   (torch.bfloat16, False, True), (torch.bfloat16, False, False)]:
+        assert step(quant, relu, grad_bias) == [[None, relu, quant, False, True, grad_bias, False, False]]
+    assert step(torch.bfloat16, True, True) == []     # the second one's graph
+
+
 @pytest.mark.parametrize("op", OPS)
 def test_saved_tensor_hooks(op):
     packed = []
