@@ -61,6 +61,16 @@ __device__ __forceinline__ float enc_value(int k, int b, float frac) {
     return k < b ? 1.0f : (k == b ? frac : 0.0f);
 }
 
+// The value at column p of sample n, whose feature is f or a later one; all
+// from global memory.
+__device__ __forceinline__ float enc_lookup(const EncArgs &a, int64_t n, int f, int p) {
+    while (f + 1 < a.F && a.offsets[f + 1] <= p) ++f;
+    const float v = a.x[n * a.F + f];
+    const float *e = a.edges + static_cast<int64_t>(f) * (a.B + 1);
+    const int b = find_bin(v, e, clamp_nbins(a.nbins[f], a.B));
+    return enc_value(p - a.offsets[f], b, (v - e[b]) * a.iw[static_cast<int64_t>(f) * a.B + b]);
+}
+
 // The group's tables and its samples' bins, shared by the two kernels.
 // TBL: edges and inverse widths in LDS (else read from global memory, see
 // plan_encode).
@@ -160,7 +170,8 @@ struct EncGroup {
 
 // V4: 16-byte stores (T a multiple of 4).  A group owns the vectors whose
 // first column is one of its features'; such a vector may end in up to three
-// features of the next group, which this one searches too.
+// features of the next group, which this one searches too (a vector that goes
+// past those, as behind features without columns, is looked up value by value).
 template <bool V4, bool TBL>
 __global__ __launch_bounds__(kEncBlock) void ple_encode_kernel(EncArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -201,6 +212,13 @@ __global__ __launch_bounds__(kEncBlock) void ple_encode_kernel(EncArgs a) {
                 const int mid = (lo + hi) >> 1;
                 if (gr.s_off[mid] <= p0) lo = mid;
                 else hi = mid;
+            }
+            if (V4 && gr.f0 + nf < a.F && p0 + W - 1 >= gr.s_off[nf]) {
+                for (int s = s0; s < ns; s += sets) {
+                    for (int j = 0; j < W; ++j)
+                        a.out[(n0 + s) * T + p0 + j] = enc_lookup(a, n0 + s, gr.f0 + lo, p0 + j);
+                }
+                continue;
             }
             int fq[W], kq[W];
             int f = lo;

@@ -76,3 +76,31 @@ def test_encode_groups(name):
     out = ops.encode(t(x), *tables, total).cpu().numpy()
     exp = po.encoding_closed_form(x, edges, inv_w, n_bins, dtype=np.float32).astype(np.float32)
     np.testing.assert_array_equal(out, exp)
+
+
+@pytest.mark.parametrize("n", [3, 700])
+@pytest.mark.parametrize("total_mod", [0, 1])
+def test_features_without_columns(n, total_mod):
+    """Runs of features with no bins (equal offsets) between the others: their
+    columns are none, and the rest is as without them, at every boundary of
+    groups and vectors."""
+    import piecewiselinearembeddings_optimized_amd  # noqa: F401
+
+    ops = torch.ops.rtdl_num_embeddings_cuda
+    rng = np.random.default_rng(5)
+    counts = np.where(rng.random(1500) < 0.8, 0, rng.integers(1, 61, 1500))
+    counts[0] = 3
+    counts[-1] = 1 + (total_mod - counts[:-1].sum() - 1) % 4
+    bins = [np.unique(rng.uniform(-2, 2, max(c, 1) + 1).astype(np.float32)) for c in counts]
+    edges, inv_w, _ = workloads.pad_bins(bins)
+    n_bins = counts.astype(np.int32)
+    x = rng.uniform(-2.5, 2.5, (n, len(counts))).astype(np.float32)
+    offs = (np.cumsum(n_bins) - n_bins).astype(np.int32)
+    total = int(n_bins.sum())
+    assert total % 4 == total_mod
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    out = ops.encode(t(x), t(edges), t(inv_w), t(n_bins), t(offs), total).cpu().numpy()
+    has = n_bins > 0
+    args = (np.ascontiguousarray(a[has]) for a in (edges, inv_w, n_bins))
+    exp = po.encoding_closed_form(np.ascontiguousarray(x[:, has]), *args, dtype=np.float32).astype(np.float32)
+    np.testing.assert_array_equal(out, exp)
