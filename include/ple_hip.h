@@ -272,8 +272,9 @@ int ple_encode_backward_launch(const float *grad_output, const float *x, const f
  * The launch plan of ple_encode_launch (backward 0) or
  * ple_encode_backward_launch (backward 1) for a shape, without launching.
  * `output` may be NULL (then taken as 16-byte aligned).  Returns the error the
- * launch would return for the sizes, else fills `info`; all zeros: the
- * backward of a small call, one thread per (sample, feature) pair.
+ * launch would return for the sizes, else fills `info`; all zeros: no feature
+ * groups, but whole rows (forward) or one thread per (sample, feature) pair
+ * (backward).
  *   features_per_group  adjacent features whose columns a workgroup writes
  *   features_searched   features whose bins it searches: with 16-byte stores up
  *                       to three more, whose columns share its last vector

@@ -14,22 +14,24 @@
 // b > 0 and x == e_b (both neighbouring clamps pass at their bounds) -- the
 // same two-term rule as the embedding's dx.
 //
-// Both kernels: one workgroup per (group of FG adjacent features, chunk of
+// By feature groups: one workgroup per (group of FG adjacent features, chunk of
 // samples).  It keeps the group's edges and inverse widths in LDS (searched
 // in global memory, a wave's 64 pairs touch up to 64 lines a step, which cost
 // more than the searches) and walks its samples in blocks of R rows; a thread
 // searches up to kEncPairs pairs of a block side by side, their x loaded a
-// block ahead.
-//
-// Forward: (b, frac) of the block's pairs go to LDS, then the threads walk
-// the group's columns of a row in 16-byte vectors -- each finds the features
-// of its columns once a block and writes them for every row -- so a store
-// instruction covers 1 KiB of one row, and the next block is searched while
-// the stores drain.  Bound by those stores, with the table set-up before them:
-// 16384 x 128, 48 bins (403 MB written) 109 -> 91 us, 700 x 900, 100 bins 366
-// -> 56.  Backward: one or two elements of g per pair, each in a line of its
+// block ahead.  Forward: (b, frac) of the block's pairs go to LDS, then the
+// threads walk the group's columns of a row in 16-byte vectors -- each finds the
+// features of its columns once a block and writes them for every row -- so a
+// store instruction covers 1 KiB of one row, and the next block is searched
+// while the stores drain.  Bound by those stores, with the table set-up before
+// them: 16384 x 128, 48 bins (403 MB written) 109 -> 91 us, 700 x 900, 100 bins
+// 366 -> 56.  Backward: one or two elements of g per pair, each in a line of its
 // own, kEncPairs lines in flight a thread and past the caches (each line is
 // read once): 74 -> 50 us and 38 -> 24 there.
+//
+// Without groups, where the tables do not repay their set-up (enc_whole_rows,
+// enc_grouped_backward): whole rows in small workgroups, forward; one thread
+// per pair, backward.
 
 #include <algorithm>
 
@@ -39,6 +41,7 @@
 namespace ple {
 namespace {
 
+constexpr int kEncRows = 8;      // samples of a workgroup by whole rows
 constexpr int kEncBlock = 2 * kBlock;
 constexpr int kEncPairs = 4;    // pairs of a block a thread searches, at most
 constexpr int kEncBlockPairs = kEncPairs * kEncBlock;
@@ -140,7 +143,9 @@ struct EncGroup {
         if constexpr (TBL) return s_iw + fl * a.B;
         else return a.iw + static_cast<int64_t>(f0 + fl) * a.B;
     }
-    // find_bin of the thread's pairs, a step of every search at a time
+    // find_bin of the thread's pairs, a step of every search at a time; in
+    // global memory until the wave's last one ends, as one feature may be much
+    // wider than the others
     __device__ __forceinline__ void find(int (&fl)[kEncPairs], int (&b)[kEncPairs]) const {
         int lo[kEncPairs], hi[kEncPairs], n[kEncPairs];
         const float *e[kEncPairs];
@@ -152,8 +157,8 @@ struct EncGroup {
             lo[u] = 0;
             hi[u] = n[u] + 1;
         }
-        const int steps = 32 - __clz(a.B + 1);
-        for (int t = 0; t < steps; ++t) {
+        auto step = [&]() __attribute__((always_inline)) {
+            bool more = false;
 #pragma unroll
             for (int u = 0; u < kEncPairs; ++u) {
                 const int mid = (lo[u] + hi[u]) >> 1;
@@ -161,12 +166,75 @@ struct EncGroup {
                 const bool below = xv[u] < e[u][min(mid, n[u])];
                 hi[u] = live && below ? mid : hi[u];
                 lo[u] = live && !below ? mid + 1 : lo[u];
+                more |= lo[u] < hi[u];
             }
+            return more;
+        };
+        if constexpr (TBL) {
+            const int steps = 32 - __clz(a.B + 1);
+            for (int t = 0; t < steps; ++t) step();
+        } else {
+            while (__any(step())) {}
         }
 #pragma unroll
         for (int u = 0; u < kEncPairs; ++u) b[u] = clamp_bin(lo[u] - 1, n[u]);
     }
 };
+
+// Forward by whole rows: one workgroup per kEncRows samples, every feature
+// searched in global memory, the threads walking the row's columns.  No set-up
+// and many small workgroups, whose searches and stores overlap each other's.
+template <bool V4>
+__global__ __launch_bounds__(kBlock) void ple_encode_rows_kernel(EncArgs a) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int F = a.F, B = a.B, T = a.T;
+    int *s_off = reinterpret_cast<int *>(lds);                 // [F + 1] column offsets
+    int *s_bin = s_off + F + 1;                                // [kEncRows][F]
+    float *s_frac = reinterpret_cast<float *>(s_bin + kEncRows * F);
+    const int tid = threadIdx.x;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kEncRows;
+    const int ns = static_cast<int>(min(static_cast<int64_t>(kEncRows), a.N - n0));
+
+    for (int i = tid; i < F; i += kBlock) s_off[i] = a.offsets[i];
+    if (tid == 0) s_off[F] = T;
+    for (int i = tid; i < ns * F; i += kBlock) {
+        const int s = i / F;
+        const int f = i - s * F;
+        const float v = a.x[(n0 + s) * F + f];
+        const int n = clamp_nbins(a.nbins[f], B);
+        const float *e = a.edges + static_cast<int64_t>(f) * (B + 1);
+        const int b = find_bin(v, e, n);
+        s_bin[i] = b;
+        s_frac[i] = (v - e[b]) * a.iw[static_cast<int64_t>(f) * B + b];
+    }
+    __syncthreads();
+
+    constexpr int W = V4 ? 4 : 1;
+    for (int p0 = tid * W; p0 < T; p0 += kBlock * W) {
+        // feature of column p0: last f with off[f] <= p0
+        int lo = 0, hi = F;          // invariant: off[lo] <= p0 < off[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (s_off[mid] <= p0) lo = mid;
+            else hi = mid;
+        }
+        int fq[W], kq[W];
+        int f = lo;
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            const int p = min(p0 + j, T - 1);
+            while (f + 1 < F && p >= s_off[f + 1]) ++f;
+            fq[j] = f;
+            kq[j] = p - s_off[f];
+        }
+        for (int s = 0; s < ns; ++s) {
+            float v[W];
+#pragma unroll
+            for (int j = 0; j < W; ++j) v[j] = enc_value(kq[j], s_bin[s * F + fq[j]], s_frac[s * F + fq[j]]);
+            store_out<PLE_DTYPE_F32, W>(a.out, (n0 + s) * T + p0, v);
+        }
+    }
+}
 
 // V4: 16-byte stores (T a multiple of 4).  A group owns the vectors whose
 // first column is one of its features'; such a vector may end in up to three
@@ -257,35 +325,34 @@ __global__ __launch_bounds__(kEncBlock) void ple_encode_kernel(EncArgs a) {
     }
 }
 
-// One thread per (sample, feature) pair, everything from global memory: small
-// calls, whose time is the round trips of one pair (3000 x 5, 256 bins: 3.8
-// us against 8.6 with staged tables; 5759 x 84, 21 bins: 9.5 against 11.1;
-// 100000 x 6, 100 bins: 23.8 against 20.6, 700 x 900: 37.6 against 23.7).
-constexpr int64_t kEncSmallPairs = 1 << 19;
-__global__ __launch_bounds__(kBlock) void ple_encode_backward_small_kernel(EncArgs a) {
+// One thread per (sample, feature) pair, everything from global memory: no
+// set-up, and the round trips of one pair for a small call (see
+// enc_grouped_backward).
+__global__ __launch_bounds__(kBlock) void ple_encode_backward_pair_kernel(EncArgs a) {
     const int F = a.F, B = a.B, T = a.T;
-    const int64_t p = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (p >= a.N * F) return;
-    const int64_t n = p / F;
-    const int f = static_cast<int>(p - n * F);
-    const float v = a.x[p];
-    const int nb = clamp_nbins(a.nbins[f], B);
-    const float *e = a.edges + static_cast<int64_t>(f) * (B + 1);
-    const float *iw = a.iw + static_cast<int64_t>(f) * B;
-    const int b = find_bin(v, e, nb);
-    // column of component b; columns outside [0, T) (offsets that do not
-    // match n_bins) read nothing
-    const int c = a.offsets[f] + b;
-    const float *grow = a.g + n * T;
-    float r = (c >= 0 && c < T) ? grow[c] * iw[b] : 0.0f;
-    if (b > 0 && v == e[b] && c - 1 >= 0 && c - 1 < T) r = fmaf(grow[c - 1], iw[b - 1], r);
-    a.out[p] = r;
+    const int64_t pairs = a.N * F;
+    for (int64_t p = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; p < pairs;
+         p += static_cast<int64_t>(gridDim.x) * kBlock) {
+        const int64_t n = p / F;
+        const int f = static_cast<int>(p - n * F);
+        const float v = a.x[p];
+        const int nb = clamp_nbins(a.nbins[f], B);
+        const float *e = a.edges + static_cast<int64_t>(f) * (B + 1);
+        const float *iw = a.iw + static_cast<int64_t>(f) * B;
+        const int b = find_bin(v, e, nb);
+        // column of component b; columns outside [0, T) (offsets that do not
+        // match n_bins) read nothing
+        const int c = a.offsets[f] + b;
+        const float *grow = a.g + n * T;
+        float r = (c >= 0 && c < T) ? grow[c] * iw[b] : 0.0f;
+        if (b > 0 && v == e[b] && c - 1 >= 0 && c - 1 < T) r = fmaf(grow[c - 1], iw[b - 1], r);
+        a.out[p] = r;
+    }
 }
 
-template <bool TBL>
 __global__ __launch_bounds__(kEncBlock) void ple_encode_backward_kernel(EncArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
-    EncGroup<TBL> gr(a, lds);
+    EncGroup<true> gr(a, lds);
     if (!gr.init(0)) return;
     const int nf = gr.nf, T = a.T;
     gr.load_x(gr.n_begin);
@@ -324,29 +391,51 @@ __global__ __launch_bounds__(kEncBlock) void ple_encode_backward_kernel(EncArgs 
     }
 }
 
+// Features whose tables fit the LDS of a group's workgroup (beside the pairs
+// of a forward's block), less the halo; 0: not one feature's.
+int64_t enc_table_features(int64_t B, int halo, bool forward) {
+    const size_t pair_bytes = forward ? 8 * static_cast<size_t>(kEncBlockPairs) : 0;
+    const size_t per_f = 4 * (2 * static_cast<size_t>(B) + 3);   // edges, inverse widths, bin count, offset
+    const size_t room = kEncLdsTarget - pair_bytes - 64;
+    return std::max<int64_t>(static_cast<int64_t>(room / per_f) - halo, 0);
+}
+
+// Entries of the tables per bin in use (all features' have the widest one's size).
+int64_t enc_padding(int64_t F, int64_t B, int64_t T) { return F * B / T; }
+
+// Whether the forward leaves tables that are mostly padding in global memory:
+// LDS would fill up with a few features' and leave groups of a few columns (817
+// x 431, one of 1422 bins among 6: 77 us with tables in LDS, 17 without).
+bool enc_global_tables(int64_t F, int64_t B, int64_t T, int halo) {
+    return F > 64 && enc_table_features(B, halo, true) < 8 && enc_padding(F, B, T) >= 8;
+}
+
 // Features a group: as many as two workgroups' LDS a CU hold (fewer where the
-// samples alone do not fill the CUs); chunks: one round of workgroups; rows a
-// block: kEncPairs pairs a thread; with the features that a row of a block has
-// never more than kEncBlockPairs, the pairs that the threads search.  halo:
-// further features a group searches.  False: a single feature's tables do not
-// fit LDS; then they stay in global memory.
+// samples alone do not fill the CUs).  Chunks: one round of workgroups, rounded
+// down (a few workgroups of a second round take as long as the first: 11297 x
+// 1744, 20 bins: 579 us rounded up, 423 down), their blocks all of one size.
+// Rows a block: kEncPairs pairs a thread at most; with the features that a row of a block has never more than
+// kEncBlockPairs, the pairs that the threads search.  halo: further features a
+// group searches.  False: the tables stay in global memory, as not one
+// feature's fit LDS, or as they are mostly padding (enc_global_tables).
 bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
     const int cus = device_cu_count();
-    const size_t pair_bytes = forward ? 8 * static_cast<size_t>(kEncBlockPairs) : 0;
-    const size_t per_f = 4 * (2 * static_cast<size_t>(a.B) + 3);   // edges, inverse widths, bin count, offset
-    const size_t room = kEncLdsTarget - pair_bytes - 64;
-    const bool tbl = per_f * (1 + halo) <= room;
-    int64_t fg = tbl ? static_cast<int64_t>(room / per_f) - halo : 512;
+    int64_t fg = enc_table_features(a.B, halo, forward);
+    const bool tbl = fg > 0 && !(forward && enc_global_tables(a.F, a.B, a.T, halo));
+    if (!tbl) fg = 512;
     fg = std::min<int64_t>({fg, a.F, kEncBlockPairs - halo});
     const int64_t rows = (a.N + 15) / 16;
     while (fg > 16 && (a.F + fg - 1) / fg * rows < cus) fg = (fg + 1) / 2;
     a.FG = static_cast<int>(std::max<int64_t>(1, fg));
     a.G = (a.F + a.FG - 1) / a.FG;
     const int nfh = std::min(a.F, a.FG + halo);
-    a.R = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kEncBlockPairs / nfh, (a.N * a.G + cus - 1) / cus)));
-    int64_t c = (2 * static_cast<int64_t>(cus) + a.G - 1) / a.G;
-    c = std::max<int64_t>(1, std::min<int64_t>(c, (a.N + a.R - 1) / a.R));
-    a.NC = ((a.N + c - 1) / c + a.R - 1) / a.R * a.R;
+    const int64_t r_max =
+        std::max<int64_t>(1, std::min<int64_t>(kEncBlockPairs / nfh, (a.N * a.G + cus - 1) / cus));
+    const int64_t c = std::max<int64_t>(1, std::min<int64_t>(2 * static_cast<int64_t>(cus) / a.G, (a.N + r_max - 1) / r_max));
+    const int64_t per = (a.N + c - 1) / c;                  // samples a chunk, in blocks of one size
+    const int64_t blocks = (per + r_max - 1) / r_max;
+    a.R = static_cast<int>((per + blocks - 1) / blocks);
+    a.NC = a.R * blocks;
     a.C = static_cast<int>((a.N + a.NC - 1) / a.NC);
     size_t off = forward ? 8 * static_cast<size_t>(a.R) * nfh : 0;
     auto take = [&](int &field, size_t bytes) {
@@ -361,8 +450,11 @@ bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
     return tbl;
 }
 
-// The most features the forward takes, part of its interface (ple_hip.h).
+// The most features the forward takes: the whole-row kernel's LDS holds every
+// feature's offset and kEncRows pairs.
+constexpr size_t enc_rows_lds_bytes(int F) { return 4 * static_cast<size_t>(F + 1) + 8 * static_cast<size_t>(kEncRows) * F; }
 constexpr int kEncMaxFeatures = 2409;
+static_assert(enc_rows_lds_bytes(kEncMaxFeatures) <= kLdsMax && enc_rows_lds_bytes(kEncMaxFeatures + 1) > kLdsMax);
 
 EncArgs enc_args(const EncodeRequest &r) {
     EncArgs a{};
@@ -388,12 +480,78 @@ int enc_launch(K kernel, const EncArgs &a, int halo, size_t lds, hipStream_t s) 
 
 }  // namespace
 
+namespace {
+
+// Whether the forward goes by whole rows instead of feature groups (either
+// way the same values; times in us, whole rows / groups).
+//  * Where LDS holds few features' tables, groups are narrow, most of all when
+//    one wide feature pads the others' tables: 16384 x 500, one of 1024 bins
+//    among 4: 149 / 890; 16384 x 64, 2 to 235 bins: 57 / 72; 10019 x 160, 217
+//    bins: 339 / 402.  Under 32 features; 16 where the row's own searches are
+//    many (10687 x 464, one of 341 bins among 11: 152 / 105) or its stores
+//    single columns (15937 x 144, one of 304 bins among 19: 90 / 74).  Few
+//    samples by whole rows leave CUs idle, which costs more (1024 x 500, 1024
+//    bins: 1180 / 610), though less than much padding does from 2048 samples
+//    on (3292 x 1074, one of 1040 bins among 10: 111 / 179; but 2339 x 382, up
+//    to 1241 bins, 241 on average: 498 / 287), and from 384 to 65536 samples
+//    of up to 128 features (444 x 49, one of 3938 bins among 22: 25 / 53; 11907
+//    x 118, one of 111 among 1: 16 / 25; but 145625 x 102, one of 96 among 2:
+//    193 / 127).
+//  * Up to 64 features, a row's searches take a round or two of a workgroup's
+//    threads and the groups' tables do not repay their set-up: 50000 x 10, 73
+//    bins: 42 / 53; 256 x 8, 48 bins: 5.2 / 7.2; at 16384 x 127, 47 bins, 142 /
+//    108.  Not where many samples have few bins, or rows too short for a
+//    workgroup (66354 x 26, 15 bins: 41 / 30; 81000 x 4, 230 columns: 30 / 23);
+//    nor for long rows of few samples (816 x 42, 530 bins: 51 / 29), of under
+//    4096 if they go by single columns (1246 x 62, 497 bins: 130 / 43), unless
+//    the tables are padding (826 x 26, one of 3012 bins among 12: 12 / 16).
+// (Launches count threads in 32 bits, kBlock for kEncRows samples.)
+bool enc_whole_rows(const EncodeRequest &r, int halo) {
+    if (r.N > (int64_t{1} << 26)) return false;
+    const bool filled = r.N >= 4096;   // two workgroups for each of 256 CUs
+    const int64_t padding = enc_padding(r.F, r.B, r.T);
+    const int64_t fit = enc_table_features(r.B, halo, true);
+    const bool narrow = r.F <= 256 && halo > 0;
+    if (filled && fit < std::min<int64_t>(r.F, narrow ? 32 : 16)) return true;
+    if (r.N >= 2048 && padding >= 8 && fit < std::min<int64_t>(r.F, narrow ? 32 : 8)) return true;
+    if (r.F <= 128 && padding >= 8 && r.N >= 384 && r.N <= 65536) return true;
+    if (r.F > 64 || (r.N > 16384 && (r.T < 256 || r.B <= 16))) return false;
+    return filled || r.T <= 1280 || r.N >= (padding >= 4 ? 768 : (halo > 0 ? 1536 : 4096));
+}
+
+// Whether the backward goes by feature groups (times in us, groups / one
+// thread per pair): from 2^21 pairs on (12509 x 324, one of 330 bins among 30:
+// 89 / 163; 270000 x 15, 2 bins: 24 / 25), from 2^20 of at least 128 features
+// (2821 x 542, one of 115 bins among 5: 22 / 33), or from 2^19 with a gradient of 64
+// MB of at least 32 features (1921 x 448, 143 bins: 26 / 44; but 117000 x 5:
+// 17 / 13, and 13 MB, 110000 x 6: 11 / 9).  Below, the tables' set-up costs
+// more than it saves (3000 x 5, 256 bins: 6.9 / 4.0), as it does where LDS holds
+// but a few features' (8000 x 158, 3220 bins: 42 / 31; none at all, 16384 x 64,
+// 8000 bins, searched from global memory: 26 / 14).
+bool enc_grouped_backward(const EncodeRequest &r) {
+    const int64_t pairs = r.N * r.F, fit = enc_table_features(r.B, 0, false);
+    if (fit == 0 || pairs < (1 << 19)) return false;
+    if (pairs >= (1 << 21)) return true;
+    if (fit < 4) return false;
+    return (r.F >= 128 && pairs >= (1 << 20)) || (r.F >= 32 && r.N * r.T >= (1 << 24));
+}
+
+}  // namespace
+
 int encode_run(const EncodeRequest &r) {
     if (r.T < 1 || r.T > INT32_MAX / 2) return PLE_E_TOO_LARGE;
     if (r.F > kEncMaxFeatures) return PLE_E_UNSUPPORTED;
     EncArgs a = enc_args(r);
     const bool v4 = enc_vectors(r);
     const int halo = v4 ? 3 : 0;
+    if (enc_whole_rows(r, halo)) {
+        const dim3 grid(static_cast<unsigned>((r.N + kEncRows - 1) / kEncRows));
+        const size_t lds = enc_rows_lds_bytes(a.F);
+        if (v4) hipLaunchKernelGGL(ple_encode_rows_kernel<true>, grid, dim3(kBlock), lds, r.stream, a);
+        else hipLaunchKernelGGL(ple_encode_rows_kernel<false>, grid, dim3(kBlock), lds, r.stream, a);
+        const hipError_t e = hipGetLastError();
+        return e == hipSuccess ? PLE_OK : static_cast<int>(e);
+    }
     size_t lds;
     const bool tbl = plan_encode(a, halo, true, lds);
     if (v4) {
@@ -407,26 +565,25 @@ int encode_run(const EncodeRequest &r) {
 int encode_backward_run(const EncodeRequest &r) {
     if (r.T < 1 || r.T > INT32_MAX / 2) return PLE_E_TOO_LARGE;
     EncArgs a = enc_args(r);
-    if (r.N * r.F < kEncSmallPairs) {
-        const int64_t blocks = (r.N * r.F + kBlock - 1) / kBlock;
-        hipLaunchKernelGGL(ple_encode_backward_small_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0,
+    if (!enc_grouped_backward(r)) {
+        const int64_t blocks = std::min((r.N * r.F + kBlock - 1) / kBlock, static_cast<int64_t>(device_cu_count()) * 32);
+        hipLaunchKernelGGL(ple_encode_backward_pair_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0,
                            r.stream, a);
         const hipError_t e = hipGetLastError();
         return e == hipSuccess ? PLE_OK : static_cast<int>(e);
     }
     size_t lds;
-    const bool tbl = plan_encode(a, 0, false, lds);
-    return tbl ? enc_launch(ple_encode_backward_kernel<true>, a, 0, lds, r.stream)
-               : enc_launch(ple_encode_backward_kernel<false>, a, 0, lds, r.stream);
+    plan_encode(a, 0, false, lds);
+    return enc_launch(ple_encode_backward_kernel, a, 0, lds, r.stream);
 }
 
 int encode_plan_info(const EncodeRequest &r, bool backward, ple_encode_plan_info_t *info) {
     if (r.T < 1 || r.T > INT32_MAX / 2) return PLE_E_TOO_LARGE;
     if (!backward && r.F > kEncMaxFeatures) return PLE_E_UNSUPPORTED;
     *info = ple_encode_plan_info_t{};
-    if (backward && r.N * r.F < kEncSmallPairs) return PLE_OK;
     EncArgs a = enc_args(r);
     const int halo = !backward && enc_vectors(r) ? 3 : 0;
+    if (backward ? !enc_grouped_backward(r) : enc_whole_rows(r, halo)) return PLE_OK;
     size_t lds;
     info->lds_tables = plan_encode(a, halo, !backward, lds) ? 1 : 0;
     info->features_per_group = a.FG;

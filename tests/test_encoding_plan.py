@@ -26,8 +26,8 @@ def test_block_holds_no_more_pairs_than_are_searched(bins, backward):
         for n in SAMPLES:
             for total in {f * bins, (f * bins + 3) // 4 * 4, max(f * bins // 2, 1)}:
                 pl = capi.encode_plan(n, f, bins, total, backward)
-                if backward and pl["groups"] == 0:
-                    continue        # one thread per pair
+                if pl["groups"] == 0:
+                    continue        # whole rows, or one thread per pair
                 assert pl["rows_per_block"] >= 1 and pl["chunks"] >= 1
                 assert pl["rows_per_block"] * pl["features_searched"] <= pl["pairs_per_block"], (n, f, total, pl)
                 assert pl["features_per_group"] * pl["groups"] >= f
@@ -36,6 +36,7 @@ def test_block_holds_no_more_pairs_than_are_searched(bins, backward):
 
 def test_forward_feature_limit():
     assert capi.encode_plan(8, 2409, 1, 2409)["groups"] >= 1
+    assert capi.encode_plan(4096, 2409, 4000, 2409 * 4000)["groups"] == 0     # whole rows: all in LDS
     with pytest.raises(capi.PleError):
         capi.encode_plan(8, 2410, 1, 2410)
     assert capi.encode_plan(300000, 2410, 1, 2410, backward=True)["groups"] >= 1

@@ -48,11 +48,14 @@ MAX_FORWARD_FEATURES = 2409
 
 @pytest.mark.parametrize("name", list(CASES))
 def test_encode_groups(name):
+    _check(*CASES[name])
+
+
+def _check(n, counts):
     assert torch.cuda.is_available(), "HIP device required"
     import piecewiselinearembeddings_optimized_amd  # noqa: F401  (registers the ops)
 
     ops = torch.ops.rtdl_num_embeddings_cuda
-    n, counts = CASES[name]
     f = len(counts)
     rng = np.random.default_rng(n)
     bins = [np.unique(rng.uniform(-2, 2, c + 1).astype(np.float32)) for c in counts]
@@ -104,3 +107,54 @@ def test_features_without_columns(n, total_mod):
     args = (np.ascontiguousarray(a[has]) for a in (edges, inv_w, n_bins))
     exp = po.encoding_closed_form(np.ascontiguousarray(x[:, has]), *args, dtype=np.float32).astype(np.float32)
     np.testing.assert_array_equal(out, exp)
+
+
+# Both sides of each line of the dispatch between feature groups and whole
+# rows (forward) or one thread per pair (backward).  ``one(big, small, f)``: one
+# wide feature among narrow ones, whose tables are padded to its size.
+def _one(big, small, f):
+    return [small] * (f // 2) + [big] + [small] * (f - f // 2 - 1)
+
+
+DISPATCH = {
+    "rows_64_features": (300, [4] * 64),
+    "groups_65_features": (300, [4] * 65),
+    "rows_16384_samples": (16384, [5] * 13),
+    "groups_16385_samples": (16385, [5] * 13),
+    "rows_256_columns": (16385, [17] * 14 + [18]),
+    "groups_255_columns": (16385, [17] * 15),
+    "groups_16_bins": (16385, [16] * 17),
+    "rows_1280_columns": (700, [40] * 32),
+    "groups_1281_columns": (700, [61] * 21),
+    "rows_4096_samples": (4096, [61] * 21),
+    "groups_4095_samples": (4095, [61] * 21),
+    "rows_31_features_fit": (4096, [204] * 66),
+    "groups_32_features_fit": (4096, [200] * 66),
+    "rows_15_features_fit": (4096, _one(470, 3, 257)),
+    "groups_16_features_fit": (4096, _one(439, 3, 257)),
+    "rows_1536_samples": (1536, [61] * 20 + [64]),
+    "groups_1535_samples": (1535, [61] * 20 + [64]),
+    "rows_768_samples": (768, _one(401, 50, 20)),
+    "groups_767_samples": (767, _one(401, 50, 20)),
+    "rows_384_samples": (384, _one(900, 21, 66)),
+    "groups_383_samples": (383, _one(900, 21, 66)),
+    "rows_65536_samples": (65536, _one(60, 1, 66)),
+    "groups_65537_samples": (65537, _one(60, 1, 66)),
+    "padded_2047": (2047, _one(1800, 5, 130)),
+    "padded_2048": (2048, _one(1800, 5, 130)),
+    "padded_whole_vectors": (500, _one(1804, 4, 130)),
+    "padded_one_row": (1, _one(1800, 5, 130)),
+    "backward_2_21_pairs": (65536, [2] * 32),
+    "backward_below_2_21_pairs": (65535, [2] * 32),
+    "backward_64_mb": (16384, [32] * 32),
+    "backward_below_64_mb": (16383, [32] * 32),
+    "backward_31_features": (16913, [33] * 31),
+    "backward_2_20_pairs": (8192, [3] * 128),
+    "backward_below_2_20_pairs": (8191, [3] * 128),
+    "backward_3_features_fit": (8200, _one(2800, 2, 64)),
+}
+
+
+@pytest.mark.parametrize("name", list(DISPATCH))
+def test_dispatch(name):
+    _check(*DISPATCH[name])
