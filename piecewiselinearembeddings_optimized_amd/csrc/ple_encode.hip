@@ -26,8 +26,7 @@
 // while the stores drain.  Bound by those stores, with the table set-up before
 // them: 16384 x 128, 48 bins (403 MB written) 109 -> 91 us, 700 x 900, 100 bins
 // 366 -> 56.  Backward: one or two elements of g per pair, each in a line of its
-// own, kEncPairs lines in flight a thread and past the caches (each line is
-// read once): 74 -> 50 us and 38 -> 24 there.
+// own, kEncPairs lines in flight a thread: 74 -> 50 us and 38 -> 24 there.
 //
 // Without groups, where the tables do not repay their set-up (enc_whole_rows,
 // enc_grouped_backward): whole rows in small workgroups, forward; one thread
@@ -350,6 +349,13 @@ __global__ __launch_bounds__(kBlock) void ple_encode_backward_pair_kernel(EncArg
     }
 }
 
+// Gradients of more bytes than this, the size of the memory-side cache, are
+// read past the caches: plain loads take 5 to 15% longer there (22201 x 203,
+// 1.6 GB: 104 us against 121).  Smaller ones may still be in that cache from
+// the kernel that wrote them, where the hint would not find them (5281 x 568,
+// 18 bins, 172 MB, just used: 58 us with it, 41 without; read cold: 58 and 57).
+constexpr int64_t kEncStreamBytes = int64_t{1} << 28;
+template <bool NT>
 __global__ __launch_bounds__(kEncBlock) void ple_encode_backward_kernel(EncArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
     EncGroup<true> gr(a, lds);
@@ -375,7 +381,8 @@ __global__ __launch_bounds__(kEncBlock) void ple_encode_backward_kernel(EncArgs 
             at[u] = n * T + c;
             edge[u] = ok[u] && b[u] > 0 && gr.xv[u] == gr.edge_row(fl[u])[b[u]] && c - 1 >= 0 && c - 1 < T;
             const bool in = ok[u] && c >= 0 && c < T;
-            const float gv = __builtin_nontemporal_load(a.g + (in ? at[u] : 0));
+            const float *gp = a.g + (in ? at[u] : 0);
+            const float gv = NT ? __builtin_nontemporal_load(gp) : *gp;
             r[u] = in ? gv * gr.iw_row(fl[u])[b[u]] : 0.0f;
         }
 #pragma unroll
@@ -574,7 +581,8 @@ int encode_backward_run(const EncodeRequest &r) {
     }
     size_t lds;
     plan_encode(a, 0, false, lds);
-    return enc_launch(ple_encode_backward_kernel, a, 0, lds, r.stream);
+    return 4 * r.N * r.T > kEncStreamBytes ? enc_launch(ple_encode_backward_kernel<true>, a, 0, lds, r.stream)
+                                           : enc_launch(ple_encode_backward_kernel<false>, a, 0, lds, r.stream);
 }
 
 int encode_plan_info(const EncodeRequest &r, bool backward, ple_encode_plan_info_t *info) {

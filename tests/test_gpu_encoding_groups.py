@@ -149,6 +149,7 @@ DISPATCH = {
     "backward_64_mb": (16384, [32] * 32),
     "backward_below_64_mb": (16383, [32] * 32),
     "backward_31_features": (16913, [33] * 31),
+    "backward_above_256_mb": (16400, [128] * 32),
     "backward_2_20_pairs": (8192, [3] * 128),
     "backward_below_2_20_pairs": (8191, [3] * 128),
     "backward_3_features_fit": (8200, _one(2800, 2, 64)),
