@@ -319,6 +319,8 @@ int ple_encode_plan_query(const void *output, int64_t N, int64_t F, int64_t B, i
  *   PLE_TUNE_BWD_MFMA       1: no matrix-core backward (the sorted path for
  *                           16-bit gradients too); 2: the matrix-core backward
  *                           for every shape it can take (also past 8 chunks)
+ *   PLE_TUNE_BWD_STREAM     1: the matrix-core backward reads its gradient with
+ *                           plain loads; 2: past the caches
  * A forced value the shape cannot take is ignored.  Returns the knob's
  * previous value, or PLE_E_BAD_SHAPE for an unknown knob.  Not synchronised
  * with launches running on other threads.
@@ -336,7 +338,8 @@ enum {
     PLE_TUNE_BWD_RB = 9,
     PLE_TUNE_BWD_WG_PER_CU = 10,
     PLE_TUNE_BWD_MFMA = 11,
-    PLE_TUNE_COUNT = 12,
+    PLE_TUNE_BWD_STREAM = 12,
+    PLE_TUNE_COUNT = 13,
 };
 int ple_set_tuning(int knob, int value);
 

@@ -25,6 +25,7 @@ DTYPE_F32, DTYPE_F16, DTYPE_BF16 = 0, 1, 2
 TUNE = {
     "FWD_FS": 0, "FWD_WG_PER_CU": 1, "FWD_FB": 2, "FWD_VEC": 3, "FWD_WIDE": 4, "BWD_SIMPLE": 5,
     "BWD_SIMPLE_GLOBAL": 6, "BWD_VEC": 7, "BWD_FS": 8, "BWD_RB": 9, "BWD_WG_PER_CU": 10, "BWD_MFMA": 11,
+    "BWD_STREAM": 12,
 }
 _DTYPE_CODES = {torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
 

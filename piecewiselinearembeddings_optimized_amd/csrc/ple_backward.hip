@@ -1127,15 +1127,17 @@ constexpr int kMfmaMaxBins = 96;   // three tiles of 32 bins
 // table loads a thread has in flight in the set-up (c4, the whole kernel:
 // 4 / 8 -> 203-204 us, 16 -> 209-211, 32 -> 213-215)
 constexpr int kTabLoads = 8;
-// Gradients of at least this many bytes stream (non-temporal loads): read
-// with plain loads they pass through the 256 MB memory-side cache, which then
-// holds neither x nor the bin indices when the next forward wants them (c4:
-// the forward after this kernel 137 -> 103 us, this kernel 199 -> 207, the
-// step 329 -> 301; 16384 x 512, d = 32: 395 -> 349; 8192 x 1024, d = 8: 225
-// -> 215).  Smaller ones leave room there, and lines that two groups'
-// workgroups share are better kept (3001 x 201, d = 24, 29 MB: 76 -> 79 us
-// when streamed; 30001 x 101, d = 8, 48 MB: no difference).
-constexpr int64_t kMfmaStreamBytes = 64 << 20;
+// Gradients of at least this many bytes stream (non-temporal loads), most of
+// the 256 MB memory-side cache.  us of a bf16 forward and this backward, plain
+// / streamed, with a new x each step: 8192 x 1024, d = 24 (403 MB) 328 / 326 and
+// with the same x each step 307 / 301, as the cache then still holds it;
+// 16384 x 512, d = 32 (537 MB) 392 / 390 and 392 / 345; 12000 x 512, d = 16 (197
+// MB) 205 / 194, or 209 / 194 if the gradient has just been written.  The
+// backward alone is up to 4% slower streamed.  Smaller gradients are better
+// found in the caches, as are lines that two groups' workgroups share: 10000 x
+// 300, d = 24 (144 MB) 140 / 143; 2048 x 1024, d = 24 (101 MB) 86 / 89; 3001 x
+// 201, d = 24 (29 MB) 56 / 57.  (PLE_TUNE_BWD_STREAM: 1 never, 2 always.)
+constexpr int64_t kMfmaStreamBytes = 192 << 20;
 constexpr int kMfmaFinLanes = 4;   // lanes of a (feature, column) in the kernel's dW / db step
 // the set-up reads a group's iw and edges one entry a thread, and clears the
 // stages 16 bytes at a time
@@ -2248,7 +2250,8 @@ void launch_mfma_nq(int nq, dim3 grid, size_t lds, hipStream_t s, const BwdArgs 
 
 template <int GD, int NBT>
 void launch_mfma(int nq, dim3 grid, size_t lds, hipStream_t s, const BwdArgs &a) {
-    if (a.N * a.F * a.D * 2 >= kMfmaStreamBytes) launch_mfma_nq<GD, NBT, true>(nq, grid, lds, s, a);
+    const int knob = tuning(PLE_TUNE_BWD_STREAM);
+    if (knob == 2 || (knob != 1 && a.N * a.F * a.D * 2 >= kMfmaStreamBytes)) launch_mfma_nq<GD, NBT, true>(nq, grid, lds, s, a);
     else launch_mfma_nq<GD, NBT, false>(nq, grid, lds, s, a);
 }
 
