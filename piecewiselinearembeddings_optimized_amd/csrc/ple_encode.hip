@@ -24,9 +24,10 @@
 // features of its columns once a block and writes them for every row -- so a
 // store instruction covers 1 KiB of one row, and the next block is searched
 // while the stores drain.  Bound by those stores, with the table set-up before
-// them: 16384 x 128, 48 bins (403 MB written) 109 -> 91 us, 700 x 900, 100 bins
-// 366 -> 56.  Backward: one or two elements of g per pair, each in a line of its
-// own, kEncPairs lines in flight a thread: 74 -> 50 us and 38 -> 24 there.
+// them: 16384 x 128, 48 bins (403 MB written) by whole rows 95 us, by groups 91;
+// 700 x 900, 100 bins 244 and 81.  Backward: one or two elements of g per pair,
+// each in a line of its own, kEncPairs lines in flight a thread: by pairs 67 and
+// 32 us there, by groups 49 and 21.
 //
 // Without groups, where the tables do not repay their set-up (enc_whole_rows,
 // enc_grouped_backward): whole rows in small workgroups, forward; one thread
@@ -421,10 +422,11 @@ bool enc_global_tables(int64_t F, int64_t B, int64_t T, int halo) {
 // samples alone do not fill the CUs).  Chunks: one round of workgroups, rounded
 // down (a few workgroups of a second round take as long as the first: 11297 x
 // 1744, 20 bins: 579 us rounded up, 423 down), their blocks all of one size.
-// Rows a block: kEncPairs pairs a thread at most; with the features that a row of a block has never more than
-// kEncBlockPairs, the pairs that the threads search.  halo: further features a
-// group searches.  False: the tables stay in global memory, as not one
-// feature's fit LDS, or as they are mostly padding (enc_global_tables).
+// Rows a block: kEncPairs pairs a thread at most; times the features of a row
+// never more than kEncBlockPairs, the pairs that the threads search.  halo:
+// further features a group searches.  False: the tables stay in global memory,
+// as not one feature's fit LDS, or as they are mostly padding
+// (enc_global_tables).
 bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
     const int cus = device_cu_count();
     int64_t fg = enc_table_features(a.B, halo, forward);
@@ -438,7 +440,8 @@ bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
     const int nfh = std::min(a.F, a.FG + halo);
     const int64_t r_max =
         std::max<int64_t>(1, std::min<int64_t>(kEncBlockPairs / nfh, (a.N * a.G + cus - 1) / cus));
-    const int64_t c = std::max<int64_t>(1, std::min<int64_t>(2 * static_cast<int64_t>(cus) / a.G, (a.N + r_max - 1) / r_max));
+    const int64_t round = 2 * static_cast<int64_t>(cus) / a.G;
+    const int64_t c = std::max<int64_t>(1, std::min(round, (a.N + r_max - 1) / r_max));
     const int64_t per = (a.N + c - 1) / c;                  // samples a chunk, in blocks of one size
     const int64_t blocks = (per + r_max - 1) / r_max;
     a.R = static_cast<int>((per + blocks - 1) / blocks);
@@ -459,7 +462,9 @@ bool plan_encode(EncArgs &a, int halo, bool forward, size_t &lds) {
 
 // The most features the forward takes: the whole-row kernel's LDS holds every
 // feature's offset and kEncRows pairs.
-constexpr size_t enc_rows_lds_bytes(int F) { return 4 * static_cast<size_t>(F + 1) + 8 * static_cast<size_t>(kEncRows) * F; }
+constexpr size_t enc_rows_lds_bytes(int F) {
+    return 4 * static_cast<size_t>(F + 1) + 8 * static_cast<size_t>(kEncRows) * F;
+}
 constexpr int kEncMaxFeatures = 2409;
 static_assert(enc_rows_lds_bytes(kEncMaxFeatures) <= kLdsMax && enc_rows_lds_bytes(kEncMaxFeatures + 1) > kLdsMax);
 
@@ -484,10 +489,6 @@ int enc_launch(K kernel, const EncArgs &a, int halo, size_t lds, hipStream_t s) 
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? PLE_OK : static_cast<int>(e);
 }
-
-}  // namespace
-
-namespace {
 
 // Whether the forward goes by whole rows instead of feature groups (either
 // way the same values; times in us, whole rows / groups).
@@ -529,9 +530,9 @@ bool enc_whole_rows(const EncodeRequest &r, int halo) {
 // Whether the backward goes by feature groups (times in us, groups / one
 // thread per pair): from 2^21 pairs on (12509 x 324, one of 330 bins among 30:
 // 89 / 163; 270000 x 15, 2 bins: 24 / 25), from 2^20 of at least 128 features
-// (2821 x 542, one of 115 bins among 5: 22 / 33), or from 2^19 with a gradient of 64
-// MB of at least 32 features (1921 x 448, 143 bins: 26 / 44; but 117000 x 5:
-// 17 / 13, and 13 MB, 110000 x 6: 11 / 9).  Below, the tables' set-up costs
+// (2821 x 542, one of 115 bins among 5: 22 / 33), or from 2^19 with a gradient
+// of 64 MB of at least 32 features (1921 x 448, 143 bins: 26 / 44; but 117000 x
+// 5: 17 / 13, and 16 MB, 110000 x 6: 11 / 9).  Below, the tables' set-up costs
 // more than it saves (3000 x 5, 256 bins: 6.9 / 4.0), as it does where LDS holds
 // but a few features' (8000 x 158, 3220 bins: 42 / 31; none at all, 16384 x 64,
 // 8000 bins, searched from global memory: 26 / 14).
